@@ -1,0 +1,620 @@
+"""The work that a program using this framework has it do, as measurable cases.
+
+A case is a dict of plain values: ``kind`` names the public entry point and the other values are its
+sizes, data type and options.  ``listed()`` holds the cases that are always measured, ``draw()`` makes
+more of the same ranges:
+
+==============  ============================================================  ===================================
+kind            entry point                                                    ranges
+==============  ============================================================  ===================================
+embed_language  ``vm["embed_language"]``                                       16..512 token ids, widths 256..2048
+embed_image     ``vm["embed_image"]``                                          28..224 pixels, 1..27 layers
+prefill         ``vm["prefill"]``                                              16..968 prefix tokens, 2..4 layers
+step            ``vm["denoise_step_kv"]``                                      16..968 prefix, 4..64 suffix tokens,
+                                                                               2..18 layers
+loop, chunk     ``vm["denoise_loop_kv"]``, ``vm["chunk"]``                     as step, 3..10 Euler steps
+joint           ``vm["denoise_step"]``                                         as prefill and step, 2..4 layers
+attention       ``mlcv_joint_attention``                                       1..64 queries, 16..1024 prefix keys
+linear          ``mlcv_linear``, ``mlcv_linear_noalloc``                       M 1..968, K 32..16384, N 16..16384
+quantize        ``get_quant("q4f16_1").quantize_weight``                       N 16..32768, K 32..16384
+dequantize      ``get_quant("q4f16_1").dequantize_weight``                     the same
+==============  ============================================================  ===================================
+
+A program keeps one model (its weights and the context bound to them) and calls it with new inputs:
+so the weights follow from the case alone, the context is kept while the same case is prepared again,
+and the inputs follow from the seed.
+"""
+
+import math
+import os
+import re
+import sys
+import zlib
+
+import torch
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "mlc-vla_amd"))
+
+VOCAB = 257_152  # rows of the PaliGemma embedding table
+EPS = 1e-6
+THETA = 10_000.0
+
+# (prefix width, prefix MLP, action width, action MLP, query heads, kv heads, head dim): the pi0.5
+# experts, the 2-layer CPU-sized model and the dummy model of the tests
+MODELS = {
+    "pi05": (2048, 16384, 1024, 4096, 8, 1, 256),
+    "tiny": (256, 1024, 128, 512, 2, 1, 64),
+    "dummy": (64, 128, 64, 128, 8, 1, 16),
+}
+
+
+def listed():
+    return [
+        # the prompt of one request: 200 padded token ids; the smallest call, launch latency
+        {"name": "embed_language", "kind": "embed_language", "model": "pi05", "tokens": 200},
+        # one camera image through the whole SigLIP So400m/14 tower (a request has three)
+        {"name": "embed_image", "kind": "embed_image", "image": 224, "patch": 14, "hidden": 1152, "inter": 4304,
+         "layers": 27, "heads": 16, "proj": 2048},
+        # a block of four prefix layers over three images and a prompt padded to 200 tokens
+        {"name": "prefill_f16", "kind": "prefill", "model": "pi05", "dtype": "float16", "quant": "", "depth": 4,
+         "prefix": 968, "valid": 800},
+        # one velocity evaluation of the whole fp16 model at the horizon that the benchmark runs
+        {"name": "step_f16", "kind": "step", "model": "pi05", "dtype": "float16", "quant": "", "depth": 18,
+         "prefix": 968, "valid": 968, "horizon": 50},
+        # the same of the quantized model at the configuration's default horizon
+        {"name": "step_q4", "kind": "step", "model": "pi05", "dtype": "float16", "quant": "q4f16_1", "depth": 18,
+         "prefix": 968, "valid": 800, "horizon": 10},
+        # a whole request after the embeddings: prefill and ten Euler steps of the whole fp16 model
+        {"name": "chunk_f16", "kind": "chunk", "model": "pi05", "dtype": "float16", "quant": "", "depth": 18,
+         "prefix": 968, "valid": 800, "horizon": 50, "steps": 10},
+        # the same of the small float32 model (float32 is the configuration's default dtype): many small launches
+        {"name": "chunk_f32_small", "kind": "chunk", "model": "tiny", "dtype": "float32", "quant": "", "depth": 2,
+         "prefix": 32, "valid": 32, "horizon": 8, "steps": 10},
+        # two prefix layers of the full-width float32 model: the largest float32 products
+        {"name": "prefill_f32", "kind": "prefill", "model": "pi05", "dtype": "float32", "quant": "", "depth": 2,
+         "prefix": 968, "valid": 800},
+        # one layer's decode attention over an fp16 cache with a padded prefix
+        {"name": "attention", "kind": "attention", "tq": 50, "heads": 8, "kv": 1, "hd": 256, "sp": 968, "ts": 50,
+         "valid": 900, "k_f32": False},
+        # a quantized decode projection in a serving loop
+        {"name": "linear_q4", "kind": "linear", "m": 50, "k": 1024, "n": 8192, "q4": True, "bias": False,
+         "noalloc": True},
+        # a prefix projection with a bias, ragged rows
+        {"name": "linear_f16", "kind": "linear", "m": 457, "k": 2048, "n": 2560, "q4": False, "bias": True,
+         "noalloc": False},
+        # quantizing a prefix layer's gate_up weights when a checkpoint is loaded
+        {"name": "quantize", "kind": "quantize", "n": 32768, "k": 2048},
+    ]
+
+
+def _log_int(rng, lo, hi, mult=1):
+    v = math.exp(rng.uniform(math.log(lo), math.log(hi)))
+    return max(lo, min(hi, int(round(v / mult)) * mult))
+
+
+def draw(rng):
+    kind = rng.choice(["embed_language", "embed_image", "prefill", "prefill", "step", "step", "loop", "chunk",
+                       "joint", "attention", "linear", "linear", "quantize", "dequantize"])
+    if kind == "embed_language":
+        return {"kind": kind, "model": rng.choice(["pi05", "tiny"]), "tokens": _log_int(rng, 16, 512)}
+    if kind == "embed_image":
+        heads, hd = rng.choice([(16, 72), (12, 64), (4, 32)])
+        return {"kind": kind, "image": 14 * rng.randint(2, 16), "patch": 14, "hidden": heads * hd,
+                "inter": rng.choice([4304, 3072, 512]), "layers": _log_int(rng, 1, 27), "heads": heads,
+                "proj": rng.choice([2048, 256])}
+    if kind in ("prefill", "step", "loop", "chunk", "joint"):
+        model = rng.choice(["pi05", "pi05", "tiny", "dummy"])
+        dtype, quant = rng.choice([("float16", ""), ("float16", ""), ("float16", "q4f16_1"), ("float32", "")])
+        if kind == "joint":
+            dtype = "float16"
+        prefix = _log_int(rng, 16, 968)
+        c = {"kind": kind, "model": model, "dtype": dtype, "quant": quant, "prefix": prefix,
+             "valid": rng.randint((prefix + 1) // 2, prefix)}
+        deep = 18 if dtype == "float16" and kind in ("step", "loop") else 2 if dtype == "float32" else 4
+        c["depth"] = rng.randint(2, deep)
+        if kind != "prefill":
+            c["horizon"] = _log_int(rng, 4, 64)
+        if kind in ("loop", "chunk"):
+            c["steps"] = rng.randint(3, 10)
+        if kind == "joint":  # every prefix token is valid there
+            c["valid"] = prefix
+        return c
+    if kind == "attention":
+        heads = rng.choice([2, 4, 8])
+        sp = _log_int(rng, 16, 1024)
+        return {"kind": kind, "tq": _log_int(rng, 1, 64), "heads": heads, "kv": rng.choice([1, 1, heads]),
+                "hd": rng.choice([64, 128, 256, 256]), "sp": sp, "ts": rng.choice([0, rng.randint(1, 64)]),
+                "valid": rng.randint((sp + 1) // 2, sp), "k_f32": rng.random() < 0.5}
+    k = _log_int(rng, 32, 16384, 32)
+    if kind == "linear":
+        n = _log_int(rng, 16, min(16384, (1 << 25) // k), 4)
+        return {"kind": kind, "m": _log_int(rng, 1, 968), "k": k, "n": n, "q4": rng.random() < 0.5,
+                "bias": rng.random() < 0.5, "noalloc": rng.random() < 0.5}
+    return {"kind": kind, "n": _log_int(rng, 16, min(32768, (1 << 26) // k)), "k": k}
+
+
+# ---- weights and inputs ------------------------------------------------------------------------
+
+
+def _gen(seed):
+    return torch.Generator(device="cuda").manual_seed(seed)
+
+
+def _weight(name, shape, dtype):
+    """A parameter as its name and shape give it: 2-D weights as of a trained projection's size."""
+    g = _gen(zlib.crc32(("%s %s" % (name, tuple(shape))).encode()))
+    w = torch.randn(tuple(shape), generator=g, device="cuda")
+    if name.startswith("vision.") and len(shape) == 2 and name.endswith(".weight"):
+        w = w.mul_(shape[1] ** -0.5)
+    elif "layer_norm" in name and name.endswith("weight") or name.endswith("post_layernorm.weight"):
+        w = w.mul_(0.1).add_(1.0)
+    elif name.endswith("norm.0.weight"):
+        w = w.mul_(0.1)
+    else:
+        w = w.mul_(0.02)
+    return w.to(dtype)
+
+
+def _quantized(w):
+    """[N, K] fp16 -> (uint32 words as int32 [N, K/8], fp16 scales [N, K/32]): groups of 32 along K."""
+    n, k = w.shape
+    f = w.float().view(n, k // 32, 32)
+    s = (f.abs().amax(-1, keepdim=True) / 7.0).half()
+    q = ((f / s.float()).half().float() + 7.0).half().float().round().clamp_(0, 14).to(torch.int64).view(n, k // 8, 8)
+    words = (q << (4 * torch.arange(8, device=w.device))).sum(-1)
+    words = torch.where(words >= 1 << 31, words - (1 << 32), words).to(torch.int32)
+    return words, s.view(n, k // 32)
+
+
+def _dequantized(words, scales):
+    """The fp16 weights that the words and scales stand for."""
+    n, kw = words.shape
+    q = (words.to(torch.int64).unsqueeze(-1) >> (4 * torch.arange(8, device=words.device))) & 15
+    q = (q.view(n, kw // 4, 32) - 7).half() * scales.unsqueeze(-1)
+    return q.view(n, kw * 8)
+
+
+def _canonical(case, name):
+    """The velocity entry points do not read the prefix expert's weights: there every layer shares one set."""
+    if case["kind"] in ("step", "loop") and (".experts.0." in name or ".mlp.0." in name or "norm.0." in name):
+        return re.sub(r"layers\.\d+\.", "layers.0.", name)
+    return name
+
+
+def _dtype(case):
+    return torch.float32 if case.get("dtype") == "float32" else torch.float16
+
+
+class _Weights:
+    """The parameters of a case by name; the quantized model's as their words and scales."""
+
+    def __init__(self, case):
+        self.case, self.kept = case, {}
+
+    def stored(self, name, shape):
+        key = _canonical(self.case, name)
+        if key not in self.kept:
+            w = _weight(key, shape, _dtype(self.case))
+            if self.case.get("quant") and len(shape) == 2:
+                w = _quantized(w)
+            self.kept[key] = w
+        return self.kept[key]
+
+
+_MODEL = {}  # the one model that is kept: (case, vm, params)
+
+
+def _model(case):
+    from mlc_vla import runtime
+    from mlc_vla.compile import compile_model
+    from mlc_vla.compile_quant import compile_model_quant
+    from mlc_vla.model.pi0.pi0_config import GemmaExpertConfig, Pi0Config, SiglipConfig
+
+    if _MODEL.get("case") == case:
+        return _MODEL["vm"], _MODEL["params"]
+    _MODEL.clear()
+    kind = case["kind"]
+    w0, f0, w1, f1, heads, kv, hd = MODELS[case.get("model", "tiny")]
+    depth = case.get("depth", 2)
+    expert = dict(depth=depth, num_heads=heads, num_kv_heads=kv, head_dim=hd)
+    kw = dict(paligemma_variant=GemmaExpertConfig(width=w0, mlp_dim=f0, **expert),
+              action_expert_variant=GemmaExpertConfig(width=w1, mlp_dim=f1, **expert), image_keys=(),
+              max_token_len=case.get("prefix", case.get("tokens", 16)), action_horizon=case.get("horizon", 10),
+              num_denoise_steps=case.get("steps", 10), dtype=case.get("dtype", "float16"))
+    if kind == "embed_image":
+        kw["siglip"] = SiglipConfig(image_size=case["image"], patch_size=case["patch"], hidden_size=case["hidden"],
+                                    intermediate_size=case["inter"], num_hidden_layers=case["layers"],
+                                    num_attention_heads=case["heads"], projection_dim=case["proj"])
+    cfg = Pi0Config(**kw)
+    functions = [kind] if kind.startswith("embed_") else \
+        ["denoise_step"] if kind == "joint" else ["prefill", "denoise_step_kv", "denoise_loop_kv"]
+    # one captured graph per chunk or loop, as a serving program asks for
+    if case.get("quant"):
+        ex, names, _, _ = compile_model_quant(cfg, "rocm", functions, case["quant"], cuda_graph=True)
+    else:
+        ex, names = compile_model(cfg, "rocm", functions=functions, cuda_graph=True)
+    vm = runtime.VirtualMachine(ex)
+    weights = _Weights(case)
+    params = []
+    for name, p in names:
+        if name.endswith(".q_weight") or name.endswith(".q_scale"):
+            base, part = name.rsplit(".", 1)
+            n, k = p.shape[0], p.shape[1] * (8 if part == "q_weight" else 32)
+            params.append(runtime.Tensor(weights.stored(base + ".weight", (n, k))[0 if part == "q_weight" else 1],
+                                         p.dtype))
+        else:
+            params.append(runtime.Tensor(weights.stored(name, p.shape), p.dtype))
+    _MODEL.update(case=dict(case), vm=vm, params=params)
+    return vm, params
+
+
+def _rope(positions, hd, offset):
+    pos = torch.arange(offset, offset + positions, dtype=torch.float64, device="cuda")
+    ang = pos[:, None] / (THETA ** ((2.0 / hd) * torch.arange(hd // 2, dtype=torch.float64, device="cuda")))
+    return torch.cos(ang), torch.sin(ang)
+
+
+def _time_embs(steps, width):
+    """sin / cos of the flow times 1, 1 - 1/steps, ... with periods from 4e-3 to 4."""
+    t = 1.0 - torch.arange(steps, dtype=torch.float64, device="cuda") / steps
+    period = 4e-3 * 1000.0 ** torch.linspace(0, 1, width // 2, dtype=torch.float64, device="cuda")
+    ang = t[:, None] * (2 * math.pi / period)
+    return torch.cat([torch.sin(ang), torch.cos(ang)], dim=1)
+
+
+def _mask(n, valid):
+    m = torch.zeros(n, device="cuda")
+    m[valid:] = -1e9
+    return m
+
+
+def _inputs(case, seed):
+    """The tensors of one call, from the seed alone."""
+    g = _gen(seed)
+
+    def randn(*shape):
+        return torch.randn(shape, generator=g, device="cuda")
+
+    kind, dt = case["kind"], _dtype(case)
+    if kind == "embed_language":
+        return {"ids": torch.randint(0, VOCAB, (1, case["tokens"]), generator=g, device="cuda", dtype=torch.int32)}
+    if kind == "embed_image":  # pixels in [-1, 1], channels last
+        return {"image": (torch.rand((1, case["image"], case["image"], 3), generator=g, device="cuda") * 2 - 1).half()}
+    if kind == "attention":
+        s = case["hd"] ** -0.25  # logits of about unit size
+        h, kv, hd, sp, ts = case["heads"], case["kv"], case["hd"], case["sp"], case["ts"]
+        kp = randn(kv, sp, hd) * s
+        return {"q": (randn(case["tq"], h * hd) * s).half(), "kp": kp if case["k_f32"] else kp.half(),
+                "vp": randn(kv, sp, hd).half(), "ks": (randn(max(ts, 1), kv * hd) * s).half(),
+                "vs": randn(max(ts, 1), kv * hd).half(), "mask": _mask(sp, case["valid"])}
+    if kind == "linear":
+        out = {"x": randn(case["m"], case["k"]).half(), "b": (0.02 * randn(case["n"])).half()}
+        w = (0.02 * randn(case["n"], case["k"])).half()
+        if case["q4"]:
+            out["qw"], out["qs"] = _quantized(w)
+        else:
+            out["w"] = w
+        return out
+    if kind == "quantize":
+        return {"w": (0.02 * randn(case["n"], case["k"])).half()}
+    if kind == "dequantize":
+        qw, qs = _quantized((0.02 * randn(case["n"], case["k"])).half())
+        return {"qw": qw, "qs": qs}
+    w0, f0, w1, f1, heads, kv, hd = MODELS[case["model"]]
+    p, t, d = case["prefix"], case.get("horizon", 10), case["depth"]
+    out = {"mask": _mask(p, case["valid"]).view(1, 1, 1, p)}
+    if kind in ("prefill", "chunk", "joint"):
+        out["prefix"] = randn(1, p, w0).to(dt)
+    else:
+        out["keys"] = randn(d, 1, kv, p, hd)
+        out["values"] = randn(d, 1, kv, p, hd).to(dt)
+    if kind != "prefill":
+        cos, sin = _rope(t, hd, case["valid"])
+        out["cos"], out["sin"] = (a.float().view(1, t, 1, hd // 2) for a in (cos, sin))
+        noise = randn(1, t, 32)
+        if kind in ("loop", "chunk"):
+            out["x0"] = noise
+            out["te"] = _time_embs(case["steps"], w1).to(dt)
+        else:
+            out["x"] = noise.to(dt)
+            out["te"] = _time_embs(10, w1)[seed % 10].view(1, w1).to(dt)
+    return out
+
+
+def prepare(case, seed):
+    case = {k: v for k, v in case.items() if k != "name"}
+    kind = case["kind"]
+    state = {"case": case, "in": _inputs(case, seed)}
+    a = state["in"]
+    if kind in ("quantize", "dequantize"):
+        from mlc_vla.quant import get_quant
+
+        state["quant"] = get_quant("q4f16_1")
+        if kind == "dequantize":
+            from mlc_vla import runtime
+
+            state["args"] = (runtime.Tensor(a["qw"], "uint32"), runtime.Tensor(a["qs"], "float16"))
+        return state
+    if kind in ("attention", "linear"):
+        from mlc_vla import _native
+
+        state["lib"] = _native
+        shape = (case["tq"], case["heads"] * case["hd"]) if kind == "attention" else (case["m"], case["n"])
+        state["out"] = torch.empty(shape, dtype=torch.float16, device="cuda")
+        return state
+    from mlc_vla import runtime
+
+    state["vm"], state["params"] = _model(case)
+    order = {"embed_language": ("ids",), "embed_image": ("image",), "prefill": ("prefix", "mask"),
+             "step": ("keys", "values", "x", "te", "cos", "sin", "mask"),
+             "loop": ("keys", "values", "x0", "te", "cos", "sin", "mask"),
+             "chunk": ("prefix", "mask", "x0", "te", "cos", "sin"), "joint": ("prefix", "x", "te")}[kind]
+    state["args"] = tuple(runtime.as_tensor(a[k]) for k in order)
+    return state
+
+
+_ENTRY = {"embed_language": "embed_language", "embed_image": "embed_image", "prefill": "prefill",
+          "step": "denoise_step_kv", "loop": "denoise_loop_kv", "chunk": "chunk", "joint": "denoise_step"}
+
+
+def run(state):
+    case, a = state["case"], state["in"]
+    kind = case["kind"]
+    if kind in _ENTRY:
+        out = state["vm"][_ENTRY[kind]](*state["args"], state["params"])
+        return [t.torch for t in out] if isinstance(out, tuple) else out.torch
+    if kind == "quantize":
+        qw, qs = state["quant"].quantize_weight(a["w"])
+        return [qw.torch, qs.torch]
+    if kind == "dequantize":
+        return state["quant"].dequantize_weight(*state["args"]).torch
+    out, stream = state["out"], torch.cuda.current_stream().cuda_stream
+    if kind == "attention":
+        ts = case["ts"]
+        state["lib"].call("mlcv_joint_attention", a["q"].data_ptr(), case["tq"], case["heads"], case["kv"], case["hd"],
+                          a["kp"].data_ptr(), int(case["k_f32"]), a["vp"].data_ptr(), case["sp"], a["mask"].data_ptr(),
+                          a["ks"].data_ptr() if ts else None, a["vs"].data_ptr() if ts else None, ts, out.data_ptr(),
+                          stream)
+        return out
+    w, qw, qs = (a[k].data_ptr() if k in a else None for k in ("w", "qw", "qs"))
+    state["lib"].call("mlcv_linear_noalloc" if case["noalloc"] else "mlcv_linear", a["x"].data_ptr(), case["m"],
+                      case["k"], w, qw, qs, a["b"].data_ptr() if case["bias"] else None, out.data_ptr(), case["n"],
+                      stream)
+    return out
+
+
+# ---- what a pass cannot do without -------------------------------------------------------------
+
+
+def _layer_work(w, f, heads, kv, hd, rows, keys, wbytes):
+    """(flops, weight bytes) of a layer's projections and MLP over `rows` tokens, and the attention's flops."""
+    lin = w * (heads + 2 * kv) * hd + heads * hd * w + 3 * w * f
+    return 2.0 * rows * lin + 4.0 * rows * keys * heads * hd, lin * wbytes
+
+
+def work(case):
+    kind = case["kind"]
+    if kind == "embed_language":
+        w0 = MODELS[case["model"]][0]
+        return {"bytes": case["tokens"] * (4 * w0 + 4), "flops": case["tokens"] * w0}
+    if kind == "embed_image":
+        h, f, n = case["hidden"], case["inter"], (case["image"] // case["patch"]) ** 2
+        pd = case["patch"] ** 2 * 3
+        lin = case["layers"] * (4 * h * h + 2 * h * f) + pd * h + h * case["proj"]
+        flops = 2.0 * n * lin + case["layers"] * 4.0 * n * n * h
+        return {"bytes": 2.0 * lin + 2.0 * (case["image"] ** 2 * 3 + n * case["proj"]), "flops": flops}
+    if kind == "attention":
+        keys, h, kv, hd, tq = case["valid"] + case["ts"], case["heads"], case["kv"], case["hd"], case["tq"]
+        kb = 4 if case["k_f32"] else 2
+        return {"bytes": 4.0 * tq * h * hd + kv * hd * (case["valid"] * (kb + 2) + case["ts"] * 4) + 4 * case["sp"],
+                "flops": 4.0 * tq * keys * h * hd}
+    if kind == "linear":
+        m, k, n = case["m"], case["k"], case["n"]
+        return {"bytes": 2.0 * m * (k + n) + n * k * (0.5 + 2 / 32 if case["q4"] else 2), "flops": 2.0 * m * k * n}
+    if kind in ("quantize", "dequantize"):
+        nk = case["n"] * case["k"]
+        return {"bytes": nk * (2 + 0.5 + 2 / 32), "flops": 4.0 * nk}
+    w0, f0, w1, f1, h, kv, hd = MODELS[case["model"]]
+    d, p, t = case["depth"], case["prefix"], case.get("horizon", 0)
+    e = 4 if case["dtype"] == "float32" else 2
+    # the prefix expert computes the large products: on the model dtype's weights, or on the quantized bytes
+    we = 0.5 + 2 / 32 if case["quant"] else e
+    flops, nbytes = 0.0, 0.0
+    if kind in ("prefill", "chunk", "joint"):  # the last layer gives its keys and values only
+        lf, lb = _layer_work(w0, f0, h, kv, hd, p, case["valid"], we)
+        flops += (d - 1) * lf + 2.0 * p * w0 * 2 * kv * hd
+        nbytes += (d - 1) * lb + w0 * 2 * kv * hd * we + p * w0 * e
+        if kind == "prefill":
+            nbytes += d * kv * p * hd * (4 + e)
+    if kind != "prefill":
+        steps = case.get("steps", 1)
+        lf, lb = _layer_work(w1, f1, h, kv, hd, t, case["valid"] + t, we)
+        mods = (2 * d + 1) * 3 * w1 * w1
+        flops += steps * (d * lf + 2.0 * t * 2 * 32 * w1 + 2.0 * (mods + 2 * w1 * w1))
+        # the weights and the cache are read once in a step; steps after the first could keep neither on chip
+        nbytes += steps * (d * lb + (2 * 32 * w1) * we + d * kv * case["valid"] * hd * (4 + e))
+        nbytes += (mods + 2 * w1 * w1) * we + steps * (t * 32 * 8)
+    return {"bytes": nbytes, "flops": flops}
+
+
+def tolerance(case):
+    kind = case["kind"]
+    if kind in ("embed_language", "quantize", "dequantize"):
+        return "exact"  # a rounding of each element by itself
+    # about four times the error against exact() (rounding in another order shows that much): a 16-bit
+    # rounding of a 32-bit sum, 16-bit probabilities besides, 32-bit sums through the layers, 16-bit layers
+    if kind == "linear":
+        return {"rel": 1e-3, "max": 8e-3}
+    if kind == "attention":
+        return {"rel": 1.5e-3, "max": 1.5e-2}
+    if case.get("dtype") == "float32":
+        return {"rel": 1e-5, "max": 1e-3}
+    return {"rel": 6e-3, "max": 6e-2}
+
+
+# ---- the same values in 64 bits, in plain torch ---------------------------------------------------
+
+
+def _lin(x, w, b=None):
+    y = x @ w.double().T.contiguous()
+    return y if b is None else y + b.double()
+
+
+def _norm(x, eps=EPS):
+    return x / torch.sqrt((x * x).mean(-1, keepdim=True) + eps)
+
+
+def _rotated(x, cos, sin):
+    """x [rows, heads, hd]: the half-split rotation."""
+    a, b = x.chunk(2, dim=-1)
+    c, s = cos[:, None, :], sin[:, None, :]
+    return torch.cat([a * c - b * s, b * c + a * s], dim=-1)
+
+
+def _attend(q, k, v, mask):
+    """q [rows, heads, hd], k / v [kv, keys, hd], mask [keys] -> [rows, heads * hd]."""
+    rows, heads, hd = q.shape
+    out = torch.empty_like(q)
+    for h in range(heads):
+        j = h // (heads // k.shape[0])
+        logits = q[:, h].contiguous() @ k[j].T.contiguous() + mask
+        out[:, h] = torch.softmax(logits, dim=-1) @ v[j].contiguous()
+    return out.reshape(rows, heads * hd)
+
+
+class _Exact:
+    def __init__(self, case, seed):
+        self.case, self.a, self.weights = case, _inputs(case, seed), _Weights(case)
+        self.w0, self.f0, self.w1, self.f1, self.h, self.kv, self.hd = MODELS[case.get("model", "tiny")]
+
+    def w(self, name, *shape):
+        w = self.weights.stored(name, shape)
+        w = _dequantized(*w) if isinstance(w, tuple) else w
+        self.weights.kept.clear()
+        return w
+
+    def heads(self, x, n):
+        return x.view(x.shape[0], n, self.hd)
+
+    def qkv(self, xn, pre, width, cos, sin):
+        nq, nkv = self.h * self.hd, self.kv * self.hd
+        q = self.heads(_lin(xn, self.w(pre + "q_proj.weight", nq, width)), self.h)
+        k = self.heads(_lin(xn, self.w(pre + "k_proj.weight", nkv, width)), self.kv)
+        v = self.heads(_lin(xn, self.w(pre + "v_proj.weight", nkv, width)), self.kv)
+        return (_rotated(q, cos, sin) * self.hd ** -0.5, _rotated(k, cos, sin).transpose(0, 1).contiguous(),
+                v.transpose(0, 1).contiguous())
+
+    def mlp(self, x, pre, width, f):
+        gu = _lin(x, self.w(pre + "gate_up_proj.weight", 2 * f, width))
+        act = torch.nn.functional.gelu(gu[:, :f], approximate="tanh") * gu[:, f:]
+        return _lin(act, self.w(pre + "down_proj.weight", width, f))
+
+    def prefill(self):
+        c = self.case
+        x, mask = self.a["prefix"][0].double(), self.a["mask"].view(-1).double()
+        cos, sin = _rope(c["prefix"], self.hd, 0)
+        keys, values = [], []
+        for i in range(c["depth"]):
+            pre = "backbone.layers.%d." % i
+            xn = _norm(x) * (1 + self.w(pre + "input_layernorm.0.weight", self.w0).double())
+            q, k, v = self.qkv(xn, pre + "self_attn.experts.0.", self.w0, cos, sin)
+            keys.append(k)
+            values.append(v)
+            if i + 1 < c["depth"]:
+                o = _attend(q, k, v, mask)
+                x = x + _lin(o, self.w(pre + "self_attn.experts.0.o_proj.weight", self.w0, self.h * self.hd))
+                xn = _norm(x) * (1 + self.w(pre + "post_attention_layernorm.0.weight", self.w0).double())
+                x = x + self.mlp(xn, pre + "mlp.0.", self.w0, self.f0)
+        return torch.stack(keys)[:, None], torch.stack(values)[:, None]
+
+    def velocity(self, x_t, te, keys, values):
+        c, w1 = self.case, self.w1
+        silu = torch.nn.functional.silu
+        cos, sin = (self.a[n].double().view(-1, self.hd // 2) for n in ("cos", "sin"))
+        mask = torch.cat([self.a["mask"].view(-1).double(), torch.zeros(c["horizon"], device="cuda")])
+        x = _lin(x_t, self.w("action_in_proj.weight", w1, 32), self.w("action_in_proj.bias", w1))
+        cond = silu(_lin(te, self.w("time_mlp_in.weight", w1, w1), self.w("time_mlp_in.bias", w1)))
+        cond = silu(_lin(cond, self.w("time_mlp_out.weight", w1, w1), self.w("time_mlp_out.bias", w1)))
+
+        def ada(x, name):
+            m = _lin(cond, self.w(name + ".weight", 3 * w1, w1), self.w(name + ".bias", 3 * w1))
+            scale, shift, gate = m.chunk(3, dim=-1)
+            return _norm(x) * (1 + scale) + shift, gate
+
+        for i in range(c["depth"]):
+            pre = "backbone.layers.%d." % i
+            xn, gate = ada(x, pre + "input_layernorm.1.modulation")
+            q, k, v = self.qkv(xn, pre + "self_attn.experts.1.", w1, cos, sin)
+            o = _attend(q, torch.cat([keys[i, 0].double(), k], 1), torch.cat([values[i, 0].double(), v], 1), mask)
+            x = x + _lin(o, self.w(pre + "self_attn.experts.1.o_proj.weight", w1, self.h * self.hd)) * gate
+            xn, gate = ada(x, pre + "post_attention_layernorm.1.modulation")
+            x = x + self.mlp(xn, pre + "mlp.1.", w1, self.f1) * gate
+        x, _ = ada(x, "backbone.final_norm.1.modulation")
+        return _lin(x, self.w("action_out_proj.weight", 32, w1), self.w("action_out_proj.bias", 32))
+
+    def image(self):
+        c = self.case
+        p, n, h, heads = c["patch"], c["image"] // c["patch"], c["hidden"], c["heads"]
+        hd = h // heads
+        img = self.a["image"][0].double()
+        patches = img.view(n, p, n, p, 3).permute(0, 2, 1, 3, 4).reshape(n * n, p * p * 3)
+
+        def lin(x, name, out, k):
+            return _lin(x, self.w(name + ".weight", out, k), self.w(name + ".bias", out))
+
+        def ln(x, name):
+            x = x - x.mean(-1, keepdim=True)
+            return _norm(x) * self.w(name + ".weight", h).double() + self.w(name + ".bias", h).double()
+
+        x = lin(patches, "vision.patch_embedding", h, p * p * 3) + \
+            self.w("vision.position_embedding", n * n, h).double()
+        zero = torch.zeros(n * n, dtype=torch.float64, device="cuda")
+        for i in range(c["layers"]):
+            pre = "vision.layers.%d." % i
+            y = ln(x, pre + "layer_norm1")
+            q, k, v = (lin(y, pre + "self_attn." + s, h, h).view(n * n, heads, hd) for s in ("q_proj", "k_proj", "v_proj"))
+            o = _attend(q * hd ** -0.5, k.transpose(0, 1).contiguous(), v.transpose(0, 1).contiguous(), zero)
+            x = x + lin(o, pre + "self_attn.out_proj", h, h)
+            u = lin(ln(x, pre + "layer_norm2"), pre + "mlp.fc1", c["inter"], h)
+            x = x + lin(torch.nn.functional.gelu(u, approximate="tanh"), pre + "mlp.fc2", h, c["inter"])
+        return lin(ln(x, "vision.post_layernorm"), "vision.multi_modal_projector", c["proj"], h)[None]
+
+
+def exact(case, seed):
+    case = {k: v for k, v in case.items() if k != "name"}
+    kind = case["kind"]
+    e = _Exact(case, seed)
+    a = e.a
+    if kind == "embed_language":
+        table = _weight("embed_tokens.weight", (VOCAB, e.w0), torch.float16)
+        return (table[a["ids"][0].long()].double() * e.w0 ** 0.5)[None]
+    if kind == "embed_image":
+        return e.image()
+    if kind == "attention":
+        q = a["q"].double().view(case["tq"], case["heads"], case["hd"])
+        k, v, mask = a["kp"].double(), a["vp"].double(), a["mask"].double()
+        if case["ts"]:
+            ks, vs = (a[n].double().view(case["ts"], case["kv"], case["hd"]).transpose(0, 1) for n in ("ks", "vs"))
+            k, v = torch.cat([k, ks], 1), torch.cat([v, vs], 1)
+            mask = torch.cat([mask, torch.zeros(case["ts"], device="cuda")])
+        return _attend(q, k, v, mask)
+    if kind == "linear":
+        w = _dequantized(a["qw"], a["qs"]) if case["q4"] else a["w"]
+        return _lin(a["x"].double(), w, a["b"] if case["bias"] else None)
+    if kind == "quantize":  # the words have no such value
+        return [None, a["w"].double().abs().view(case["n"], -1, 32).amax(-1) / 7]
+    if kind == "dequantize":
+        n, k = case["n"], case["k"]
+        q = (a["qw"].to(torch.int64).unsqueeze(-1) >> (4 * torch.arange(8, device="cuda"))) & 15
+        return ((q.view(n, k // 32, 32) - 7).double() * a["qs"].double().unsqueeze(-1)).view(n, k)
+    if kind == "prefill":
+        return list(e.prefill())
+    if kind == "joint":
+        a["cos"], a["sin"] = (t.view(1, -1, 1, e.hd // 2) for t in _rope(case["horizon"], e.hd, case["prefix"]))
+    keys, values = e.prefill() if kind in ("chunk", "joint") else (a["keys"], a["values"])
+    if kind in ("step", "joint"):
+        return e.velocity(a["x"][0].double(), a["te"].double(), keys, values)[None]
+    x = a["x0"][0].double()
+    for i in range(case["steps"]):
+        x = x - e.velocity(x, a["te"][i:i + 1].double(), keys, values) / case["steps"]
+    return x[None]
