@@ -10,7 +10,7 @@ kind            entry point                                                    r
 embed_language  ``vm["embed_language"]``                                       16..512 token ids, widths 256..2048
 embed_image     ``vm["embed_image"]``                                          28..224 pixels, 1..27 layers
 prefill         ``vm["prefill"]``                                              16..968 prefix tokens, 2..4 layers
-step            ``vm["denoise_step_kv"]``                                      16..968 prefix, 4..64 suffix tokens,
+step            ``vm["denoise_step_kv"]``                                      16..968 prefix, 4..63 suffix tokens,
                                                                                2..18 layers
 loop, chunk     ``vm["denoise_loop_kv"]``, ``vm["chunk"]``                     as step, 3..10 Euler steps
 joint           ``vm["denoise_step"]``                                         as prefill and step, 2..4 layers
@@ -113,7 +113,7 @@ def draw(rng):
         deep = 18 if dtype == "float16" and kind in ("step", "loop") else 2 if dtype == "float32" else 4
         c["depth"] = rng.randint(2, deep)
         if kind != "prefill":
-            c["horizon"] = _log_int(rng, 4, 64)
+            c["horizon"] = _log_int(rng, 4, 63)
         if kind in ("loop", "chunk"):
             c["steps"] = rng.randint(3, 10)
         if kind == "joint":  # every prefix token is valid there
