@@ -1283,7 +1283,6 @@ int mlcv_create(const mlcv_config* cfg, mlcv_ctx** out) {
       {tiles(W1, tile_down(c).tr), c.F1, mb_t * tile_down(c).mg, tile_down(c).tr, tile_down(c).splits},
       {tiles(W1, 16), W1, mb_s, 16, c.tilings.tmlp.splits},                      // time mlp
       {tiles(W1, 64), W1, mb_s, 64, 0},
-      {std::max(2, c.NM - 2) * tiles(3 * W1, 64), W1, mb_s, 64, 0},              // modulation pieces
       {std::max(2, c.NM) * tiles(3 * W1, 16), W1, mb_s, 16, MOD_SPLITS},
       {tiles(W1, TR_AIN), c.A, mb_t, TR_AIN, SPLIT_AIN},                         // action_in
       {tiles(c.A, tile_head(c).tr), W1, mb_t * tile_head(c).mg, tile_head(c).tr, tile_head(c).splits},  // action_out
@@ -1293,6 +1292,8 @@ int mlcv_create(const mlcv_config* cfg, mlcv_ctx** out) {
     c.skws_floats = std::max(c.skws_floats, sk_ws_floats(s.ntiles, s.mb, p, s.tr));
     c.ncounters = std::max(c.ncounters, (size_t)s.ntiles * s.mb);
   }
+  const size_t mod_ws = sk_mod_ws_floats(c.NM, W1, mb_s);  // the modulation pieces on 64-row tiles
+  c.skws_floats = std::max(c.skws_floats, mod_ws);
   ALLOC(c.skws, c.skws_floats);
   ALLOC(c.counters, c.ncounters);
   {
@@ -1300,8 +1301,7 @@ int mlcv_create(const mlcv_config* cfg, mlcv_ctx** out) {
     // 64-row tiles the planner's
     const int segs = std::max(2, c.NM - 2);
     const int nt = segs * tiles(3 * W1, 16);
-    const SkPlan p = sk_plan(segs * tiles(3 * W1, 64), W1, mb_s, 0);
-    ALLOC(c.skws_side, std::max<size_t>(1, sk_ws_floats(segs * tiles(3 * W1, 64), mb_s, p, 64)));
+    ALLOC(c.skws_side, std::max<size_t>(1, mod_ws));
     ALLOC(c.counters_side, (size_t)nt * mb_s);
     c.ncounters_side = (size_t)nt * mb_s;
   }

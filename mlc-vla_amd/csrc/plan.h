@@ -67,6 +67,19 @@ inline size_t sk_ws_floats(int ntiles, int mblocks, const SkPlan& p, int tr) {
   return p.splitk > 1 ? (size_t)ntiles * mblocks * p.splitk * tr * 64 : 0;
 }
 
+// fp32 partials of the modulation pieces on 64-row tiles (T >= 64 or more than 16 steps): layer
+// 0's two norms, then the other NM - 2, of 3 W1 rows each.  The smaller piece takes more K slices,
+// so either can need the larger workspace (at W1 = 1024: 96 tiles in 3 slices against none).
+inline size_t sk_mod_ws_floats(int NM, int W1, int mblocks) {
+  const int per = (3 * W1 + 63) / 64;
+  size_t n = 0;
+  for (int segs : {2, NM - 2}) {
+    if (segs <= 0) continue;
+    n = std::max(n, sk_ws_floats(segs * per, mblocks, sk_plan(segs * per, W1, mblocks, 0), 64));
+  }
+  return n;
+}
+
 // ---- prefill tile GEMM, 256-row tiles (gemm_tile.hip) -------------------------------------
 constexpr int TG_BM = 256, TG_BK = 64, TG_NXCD = 8;
 

@@ -81,6 +81,23 @@ static void check_skinny() {
         }
 }
 
+// The modulation pieces of mlcv_bind_params on 64-row tiles (layer 0's two norms, then the other
+// NM - 2, 3 W1 rows each): the workspace mlcv_create allocates holds the partials of each piece.
+static void check_modulations() {
+  for (int D : {1, 2, 3, 4, 11, 18})
+    for (int W1 : {64, 128, 256, 1024, 2048})
+      for (int mblocks : {1, 2}) {
+        const int NM = 2 * D + 1, per = (3 * W1 + 63) / 64;
+        const size_t ws = sk_mod_ws_floats(NM, W1, mblocks);
+        for (int segs : {2, NM - 2}) {
+          ++checked;
+          const SkPlan p = sk_plan(segs * per, W1, mblocks, 0);
+          const size_t end = p.splitk > 1 ? (size_t)segs * per * mblocks * p.splitk * 64 * 64 : 0;
+          CHECK(end <= ws, "D %d W1 %d: a piece of %d norms needs %zu floats of %zu", D, W1, segs, end, ws);
+        }
+      }
+}
+
 static void check_tile() {
   for (int cus : {8, 80, 256, 304})
     for (int M : {1, 32, 255, 256, 257, 968, 4096})
@@ -140,6 +157,7 @@ static void check_tile() {
 int main() {
   check_attn();
   check_skinny();
+  check_modulations();
   check_tile();
   std::printf("plans checked: %ld, failures: %d\n", checked, failures);
   return failures ? 1 : 0;

@@ -464,3 +464,32 @@ def test_full_size_step_vs_oracle():
     ref = O.denoise_step_kv(p32, d, keys, values, x_t, te, cos, sin, pm, F32)
     _tol(got, ref)
     assert len(names) == 335
+
+
+@pytest.mark.parametrize("horizon", [64, 70])
+def test_long_horizon_step_vs_oracle(horizon):
+    """denoise_step_kv at the pi0.5 widths from 64 suffix tokens on (row-major operands, the
+    modulations in two pieces on 64-row tiles whose first splits K), 2 layers, against the float32
+    oracle."""
+    from mlc_vla.model.pi0.pi0_config import GemmaExpertConfig
+
+    expert = dict(depth=2, num_heads=8, num_kv_heads=1, head_dim=256)
+    cfg = Pi0Config(paligemma_variant=GemmaExpertConfig(width=256, mlp_dim=512, **expert),
+                    action_expert_variant=GemmaExpertConfig(width=1024, mlp_dim=4096, **expert), image_keys=(),
+                    max_token_len=48, action_horizon=horizon, dtype="float16")
+    print(f"long horizon T={horizon}", flush=True)
+    d = O.dims_from_config(cfg)
+    runner = PiZeroRunner(cfg, "rocm")
+    p16 = O.make_params(O.param_specs(d), 4, "float16")
+    params = runner.to_params([p16[n] for n, _ in runner.named_params])
+    rng = np.random.default_rng(horizon)
+    keys = rng.standard_normal((2, 1, 1, 48, 256)).astype(np.float32)
+    values = rng.standard_normal((2, 1, 1, 48, 256)).astype(np.float16)
+    x_t = rng.standard_normal((1, horizon, 32)).astype(np.float16)
+    te = O.sinusoidal_time_emb(0.7, 1024).astype(np.float16)
+    pm = make_prefix_mask_np(48, num_valid=42)
+    cos, sin = make_rope_np(horizon, 256, 10_000.0, offset=42)
+    dv = lambda a: runtime.tensor(a, runner.dev)  # noqa: E731
+    got = runner.vm["denoise_step_kv"](dv(keys), dv(values), dv(x_t), dv(te), dv(cos), dv(sin), dv(pm), params).numpy()
+    p32 = {n: v.astype(np.float32) for n, v in p16.items()}
+    _tol(got, O.denoise_step_kv(p32, d, keys, values, x_t, te, cos, sin, pm, F32))
