@@ -7,16 +7,18 @@
 // logits, softmax and probabilities (:97-122), GeGLU (:125-135) and the gated residual (:91-94)
 // round after each op, and the Euler update is x + dt * v in fp32 (pi0_model.py:165-194).
 //
-// These kernels are generic and simple (one tiled FMA GEMM, one workgroup per row or per query
-// row and head elsewhere): the float32 model is for parity at small shapes; the fp16 and q4f16_1
-// models are the fast paths.  Elementwise kernels keep the reference's rounding order
-// (floating-point contraction is off in this file; the GEMM's and the dot products' fmaf are
-// explicit).
+// The linears run on the fp32 matrix cores with the norms in their loaders and RoPE, cache writes,
+// GeGLU and residuals in their epilogues (gemm_f32.hip), where widths, head dim and pointers allow
+// (F32Model::fast); the general kernels here (one tiled FMA GEMM, one workgroup per row or per query
+// row and head elsewhere) take everything else.  Elementwise arithmetic keeps the reference's rounding
+// order (floating-point contraction is off in these files; explicit fmaf in the general GEMM and dot
+// products).
 #include <cmath>
 #include <memory>
 #include <vector>
 
 #include "../../include/mlcvla.h"
+#include "f32.h"
 #include "kernels.h"
 
 #pragma clang fp contract(off)
@@ -240,6 +242,9 @@ struct F32Model {
   int W0, F0, W1, F1, D, H, KV, HD, P, T, A, S;
   float eps;
   bool bound = false;
+  // the matrix-core kernels (gemm_f32.hip) take these widths and weight pointers; else the general ones
+  bool shape_ok = false, fast = false;
+  F32Tab* tab = nullptr;  // the 2 D + 1 modulations' weights and biases (device)
   std::vector<F32Layer> layers;
   F32Lin final_mod, ain, aout, tin, tout;
   std::vector<void*> owned;
@@ -253,6 +258,7 @@ struct F32Model {
 
   ~F32Model() {
     for (void* p : owned) (void)hipFree(p);
+    if (tab) (void)hipFree(tab);
   }
   int alloc(float** p, size_t n) {
     MLCV_HIP(hipMalloc(reinterpret_cast<void**>(p), std::max<size_t>(n, 1) * sizeof(float)));
@@ -291,8 +297,139 @@ int residual(float* x, const float* y, const float* gate, int W, int rows, hipSt
   return 0;
 }
 
-// one velocity evaluation on x_t (the model's x) with the time embedding te (pi0_model.py:142-163)
-int f32_step_on(F32Model& m, const float* keys, const float* values, const float* x_t, const float* te,
+bool f32_aligned(std::initializer_list<const void*> ps) {
+  for (const void* p : ps)
+    if ((reinterpret_cast<uintptr_t>(p) & 15) != 0) return false;
+  return true;
+}
+
+F32Op lin_op(const float* x, int ldx, int M, const F32Lin& l, int epi, float* out, int ldo) {
+  F32Op a{};
+  a.x = x;
+  a.ldx = ldx;
+  a.M = M;
+  a.K = l.K;
+  a.N = l.N;
+  a.w[0] = l.w;
+  a.b = l.b;
+  a.epi = epi;
+  a.out = out;
+  a.ldo = ldo;
+  return a;
+}
+
+// q, k and v of one expert over its rows in one product: q roped and scaled to q [M][nq], k roped and v
+// to element (m, head, d) at m * kv_m + head * kv_h + d.  with_q false: k and v alone.
+F32Op qkv_op(const F32Model& m, const F32Lin& q, const F32Lin& k, const F32Lin& v, bool with_q, const float* x, int M,
+             float* qo, float* ko, float* vo, int kv_m, size_t kv_h, const float* cs, const float* sn) {
+  F32Op a{};
+  a.x = x;
+  a.ldx = a.K = k.K;
+  a.M = M;
+  a.nq = with_q ? q.N : 0;
+  a.nkv = k.N;
+  a.N = a.nq + 2 * a.nkv;
+  a.w[0] = q.w;
+  a.w[1] = k.w;
+  a.w[2] = v.w;
+  a.epi = FE_QKV;
+  a.qo = qo;
+  a.ko = ko;
+  a.vo = vo;
+  a.hd = m.HD;
+  a.kv_m = kv_m;
+  a.kv_h = kv_h;
+  a.cos = cs;
+  a.sin = sn;
+  a.qscale = 1.0f / std::sqrt((float)m.HD);
+  a.eps = m.eps;
+  return a;
+}
+
+// the time MLP and every modulation of `steps` time embeddings te [steps][W1] into mods
+// [steps][2 D + 1][3 W1]
+int f32_mods(F32Model& m, const float* te, int steps, hipStream_t st) {
+  const int W1 = m.W1, nm = 2 * m.D + 1;
+  F32Op a = lin_op(te, W1, steps, m.tin, FE_STORE, m.tmp, W1);
+  a.act = 1;
+  MLCV_TRY(f32_gemm_launch(a, st));
+  a = lin_op(m.tmp, W1, steps, m.tout, FE_STORE, m.cond, W1);
+  a.act = 1;
+  MLCV_TRY(f32_gemm_launch(a, st));
+  a = lin_op(m.cond, W1, steps, m.final_mod, FE_STORE, m.mods, nm * 3 * W1);
+  a.tab = m.tab;
+  a.ntab = nm;
+  a.tab_stride = (size_t)3 * W1;
+  return f32_gemm_launch(a, st);
+}
+
+// one velocity evaluation of x_t with the modulations mods [2 D + 1][3 W1]: into v_out, or (x32
+// non-null) the Euler update x32 += dt * v
+int f32_velocity(F32Model& m, const float* keys, const float* values, const float* x_t, const float* mods,
+                 const float* cs, const float* sn, const float* pmask, float* v_out, float* x32, float dt,
+                 hipStream_t st) {
+  const int T = m.T, W1 = m.W1, nq = m.H * m.HD, nkv = m.KV * m.HD;
+  const size_t kvs = (size_t)m.KV * m.P * m.HD;
+  MLCV_TRY(f32_gemm_launch(lin_op(x_t, m.A, T, m.ain, FE_STORE, m.x, W1), st));
+  for (int L = 0; L < m.D; ++L) {
+    const F32Layer& ly = m.layers[L];
+    const float* mi = mods + (size_t)(2 * L) * 3 * W1;
+    const float* mp = mi + 3 * W1;
+    F32Op a = qkv_op(m, ly.q[1], ly.k[1], ly.v[1], true, m.x, T, m.q, m.k, m.v, nkv, m.HD, cs, sn);
+    a.mod = mi;
+    a.xn = m.xn;
+    MLCV_TRY(f32_gemm_launch(a, st));
+    MLCV_TRY(attn(m.q, nq, m, keys + L * kvs, values + L * kvs, m.P, pmask, m.k, m.v, nkv, T, m.attn, T, st));
+    a = lin_op(m.attn, nq, T, ly.o[1], FE_RES, m.x, W1);
+    a.gate = mi + 2 * W1;
+    MLCV_TRY(f32_gemm_launch(a, st));
+    a = lin_op(m.x, W1, T, ly.gu[1], FE_GEGLU, m.h, m.F1);
+    a.F = m.F1;
+    a.mod = mp;
+    a.xn = m.xn;
+    a.eps = m.eps;
+    MLCV_TRY(f32_gemm_launch(a, st));
+    a = lin_op(m.h, m.F1, T, ly.dn[1], FE_RES, m.x, W1);
+    a.gate = mp + 2 * W1;
+    MLCV_TRY(f32_gemm_launch(a, st));
+  }
+  F32Op a = lin_op(m.x, W1, T, m.aout, x32 ? FE_EULER : FE_STORE, x32 ? x32 : v_out, m.A);
+  a.mod = mods + (size_t)(2 * m.D) * 3 * W1;
+  a.xn = m.xn;
+  a.eps = m.eps;
+  a.dt = dt;
+  return f32_gemm_launch(a, st);
+}
+
+// the prefix layers over px; the last one gives its keys and values only (nothing reads the rest)
+int f32_prefix(F32Model& m, float* keys, float* values, hipStream_t st) {
+  const int P = m.P, W0 = m.W0, nq = m.H * m.HD;
+  const size_t kvs = (size_t)m.KV * P * m.HD;
+  for (int L = 0; L < m.D; ++L) {
+    const F32Layer& ly = m.layers[L];
+    const bool last = L == m.D - 1;
+    float *kL = keys + L * kvs, *vL = values + L * kvs;
+    F32Op a = qkv_op(m, ly.q[0], ly.k[0], ly.v[0], !last, m.px, P, m.pq, kL, vL, m.HD, (size_t)P * m.HD, m.pcos, m.psin);
+    a.nw = ly.ln_in0;
+    a.xn = m.pxn;
+    MLCV_TRY(f32_gemm_launch(a, st));
+    if (last) break;
+    MLCV_TRY(attn(m.pq, nq, m, kL, vL, P, m.mask, nullptr, nullptr, 0, 0, m.pattn, P, st));
+    MLCV_TRY(f32_gemm_launch(lin_op(m.pattn, nq, P, ly.o[0], FE_RES, m.px, W0), st));
+    a = lin_op(m.px, W0, P, ly.gu[0], FE_GEGLU, m.ph, m.F0);
+    a.F = m.F0;
+    a.nw = ly.ln_post0;
+    a.xn = m.pxn;
+    a.eps = m.eps;
+    MLCV_TRY(f32_gemm_launch(a, st));
+    MLCV_TRY(f32_gemm_launch(lin_op(m.ph, m.F0, P, ly.dn[0], FE_RES, m.px, W0), st));
+  }
+  return 0;
+}
+
+// The general form of one velocity evaluation, for widths or pointers the matrix-core kernels do not
+// take: x_t (the model's x) with the time embedding te (pi0_model.py:142-163)
+int f32_step_general(F32Model& m, const float* keys, const float* values, const float* x_t, const float* te,
                 const float* cs, const float* sn, const float* pmask, float* v_out, hipStream_t st) {
   const int T = m.T, W1 = m.W1, nq = m.H * m.HD, nkv = m.KV * m.HD, W3 = 3 * W1;
   const size_t kvs = (size_t)m.KV * m.P * m.HD;  // one layer's cache slice
@@ -347,6 +484,8 @@ int f32_create(const ::mlcv_config& cfg, F32Model** out) {
   m->A = cfg.action_dim;
   m->S = cfg.num_steps;
   m->eps = cfg.rms_norm_eps;
+  m->shape_ok = (m->HD == 16 || m->HD == 32 || m->HD == 64 || m->HD == 128 || m->HD == 256) && m->W0 % 8 == 0 &&
+                m->F0 % 8 == 0 && m->W1 % 8 == 0 && m->F1 % 8 == 0 && m->A % 8 == 0;
   MLCV_REQUIRE(m->HD % 2 == 0 && m->H % m->KV == 0, "float32 model: head_dim even, heads a multiple of kv heads");
   MLCV_REQUIRE((size_t)(m->HD + m->P + m->T) * 4 <= 64 * 1024, "float32 model: prefix_len + suffix_len too large");
   const size_t P = m->P, T = m->T, nq = (size_t)m->H * m->HD, nkv = (size_t)m->KV * m->HD;
@@ -416,6 +555,16 @@ int f32_bind(F32Model& m, const void* const* ptrs, int count) {
   lin(m.tout, m.W1, m.W1, true);
   MLCV_REQUIRE(idx == count, "internal: float32 parameter walk mismatch");
   for (int i = 0; i < count; ++i) MLCV_REQUIRE(ptrs[i] != nullptr, "null parameter pointer");
+  m.fast = m.shape_ok;
+  for (int i = 0; i < count; ++i) m.fast = m.fast && f32_aligned({ptrs[i]});
+  if (m.fast) {
+    std::vector<F32Tab> tab;
+    for (const F32Layer& ly : m.layers)
+      for (const F32Lin* l : {&ly.mod_in, &ly.mod_post}) tab.push_back({l->w, l->b});
+    tab.push_back({m.final_mod.w, m.final_mod.b});
+    if (!m.tab) MLCV_HIP(hipMalloc(reinterpret_cast<void**>(&m.tab), tab.size() * sizeof(F32Tab)));
+    MLCV_HIP(hipMemcpy(m.tab, tab.data(), tab.size() * sizeof(F32Tab), hipMemcpyHostToDevice));
+  }
   m.bound = true;
   return 0;
 }
@@ -430,6 +579,7 @@ int f32_prefill(F32Model& m, const void* prefix_embs, const float* prefix_mask, 
   const float scale = 1.0f / std::sqrt((float)m.HD);
   MLCV_HIP(hipMemcpyAsync(m.px, prefix_embs, (size_t)P * W0 * 4, hipMemcpyDeviceToDevice, st));
   MLCV_HIP(hipMemcpyAsync(m.mask, prefix_mask, (size_t)P * 4, hipMemcpyDeviceToDevice, st));
+  if (m.fast && f32_aligned({keys, values})) return f32_prefix(m, keys, vals, st);
   for (int L = 0; L < m.D; ++L) {
     const F32Layer& ly = m.layers[L];
     MLCV_TRY(norm(m.px, W0, ly.ln_in0, nullptr, m.eps, m.pxn, P, st));
@@ -456,8 +606,13 @@ int f32_prefill(F32Model& m, const void* prefix_embs, const float* prefix_mask, 
 int f32_step(F32Model& m, const float* keys, const void* values, const void* x_t, const void* time_emb,
              const float* cs, const float* sn, const float* prefix_mask, float* v_out, hipStream_t st) {
   MLCV_REQUIRE(m.bound, "parameters not bound");
-  return f32_step_on(m, keys, reinterpret_cast<const float*>(values), reinterpret_cast<const float*>(x_t),
-                     reinterpret_cast<const float*>(time_emb), cs, sn, prefix_mask, v_out, st);
+  const float* vals = reinterpret_cast<const float*>(values);
+  const float *x = reinterpret_cast<const float*>(x_t), *te = reinterpret_cast<const float*>(time_emb);
+  if (m.fast && f32_aligned({keys, vals, x, te, cs, sn, v_out})) {
+    MLCV_TRY(f32_mods(m, te, 1, st));
+    return f32_velocity(m, keys, vals, x, m.mods, cs, sn, prefix_mask, v_out, nullptr, 0.f, st);
+  }
+  return f32_step_general(m, keys, vals, x, te, cs, sn, prefix_mask, v_out, st);
 }
 
 // N Euler steps x <- x + (-1/N) v(x), x fed to each step as the model's x (pi0_model.py:165-194)
@@ -467,10 +622,16 @@ int f32_loop(F32Model& m, const float* keys, const void* values, const float* x0
   const int n = m.T * m.A;
   const float dt = (float)(-1.0 / m.S);
   MLCV_HIP(hipMemcpyAsync(m.x32, x0, (size_t)n * 4, hipMemcpyDeviceToDevice, st));
+  const float* vals = reinterpret_cast<const float*>(values);
+  const float* te = reinterpret_cast<const float*>(time_embs);
+  const bool fast = m.fast && f32_aligned({keys, vals, te, cs, sn});
   for (int i = 0; i < m.S; ++i) {
-    MLCV_TRY(f32_step_on(m, keys, reinterpret_cast<const float*>(values), m.x32,
-                         reinterpret_cast<const float*>(time_embs) + (size_t)i * m.W1, cs, sn, prefix_mask, m.vout,
-                         st));
+    if (fast) {
+      MLCV_TRY(f32_mods(m, te + (size_t)i * m.W1, 1, st));
+      MLCV_TRY(f32_velocity(m, keys, vals, m.x32, m.mods, cs, sn, prefix_mask, nullptr, m.x32, dt, st));
+      continue;
+    }
+    MLCV_TRY(f32_step_general(m, keys, vals, m.x32, te + (size_t)i * m.W1, cs, sn, prefix_mask, m.vout, st));
     f32_euler_kernel<<<ew_grid(n), 256, 0, st>>>(m.x32, m.vout, dt, n);
     MLCV_HIP(hipGetLastError());
   }

@@ -1,0 +1,81 @@
+"""The float32 model's kernels against the float32 oracle over the shapes where their tiles, slabs and
+loaders have edges: prefill K/V, one velocity, and the device loop, on random weights."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import cosine
+from mlc_vla import runtime
+from mlc_vla.model.pi0 import Pi0Config
+from mlc_vla.model.pi0.pi0_config import GemmaExpertConfig
+from mlc_vla.sample import PiZeroRunner, make_prefix_mask_np, make_rope_np, make_time_embs
+from oracle import pi0_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _tol(got, ref, what):
+    """float32 sums in another order: the tolerance of the float32 fixtures (test_gpu_golden.py)."""
+    got, ref = np.asarray(got, np.float64), np.asarray(ref, np.float64)
+    assert np.all(np.isfinite(got)), what
+    np.testing.assert_allclose(got, ref, rtol=2e-4, atol=2e-5 * float(np.abs(ref).max()), err_msg=what)
+    assert cosine(got, ref) >= 0.9999999, (what, cosine(got, ref))
+
+
+# W0, F0, W1, F1, heads, kv heads, head dim, P, valid, T, offset: offset 1 makes every pointer 4 bytes
+# off its 16-byte alignment
+SHAPES = [
+    (64, 128, 64, 128, 8, 1, 16, 31, 31, 1, 0),       # one row, one slab
+    (64, 128, 64, 128, 8, 1, 16, 33, 20, 17, 0),      # a second m tile with one row
+    (72, 136, 40, 104, 2, 2, 32, 65, 50, 33, 0),      # widths of 8 (half slabs, K tails), 3 m tiles
+    (256, 1024, 128, 512, 2, 1, 64, 130, 100, 64, 0), # 4 whole m tiles, a third m group in the prefix
+    (64, 4096, 64, 512, 1, 1, 128, 100, 77, 70, 0),   # 64 x 64 tiles (128 n tiles x 2 m tiles), T > 64
+    (64, 16384, 64, 64, 1, 1, 256, 150, 150, 5, 0),   # 128 x 128 tiles (256 x 2), a partial m tile
+    (100, 60, 36, 52, 3, 1, 20, 40, 33, 6, 0),        # widths and head dim only the general kernels take
+    (64, 128, 64, 128, 2, 1, 32, 40, 33, 6, 1),       # misaligned weights and inputs
+]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "-".join(map(str, s)))
+def test_f32_model_vs_oracle(shape):
+    w0, f0, w1, f1, heads, kv, hd, P, valid, T, off = shape
+    print(f"float32 model {shape}", flush=True)
+    expert = dict(depth=2, num_heads=heads, num_kv_heads=kv, head_dim=hd)
+    cfg = Pi0Config(paligemma_variant=GemmaExpertConfig(width=w0, mlp_dim=f0, **expert),
+                    action_expert_variant=GemmaExpertConfig(width=w1, mlp_dim=f1, **expert), image_keys=(),
+                    max_token_len=P, action_horizon=T, action_dim=32, num_denoise_steps=3, dtype="float32")
+    d = O.dims_from_config(cfg)
+    runner = PiZeroRunner(cfg, "rocm")
+    p = O.make_params(O.param_specs(d), sum(shape), "float32")
+
+    def dev(a):
+        a = np.ascontiguousarray(a, np.float32)
+        if not off:
+            return runtime.tensor(a, runner.dev)
+        flat = runtime.tensor(np.concatenate([np.zeros(1, np.float32), a.ravel()]), runner.dev)
+        return runtime.Tensor(flat.torch[1:].view(a.shape), "float32")
+
+    params = [dev(p[n]) for n, _ in runner.named_params]
+    rng = np.random.default_rng(P + T)
+    prefix = rng.standard_normal((1, P, w0)).astype(np.float32)
+    x = rng.standard_normal((1, T, 32)).astype(np.float32)
+    pm = make_prefix_mask_np(P, num_valid=valid)
+    cos, sin = make_rope_np(T, hd, 10_000.0, offset=valid)
+    te = np.concatenate(make_time_embs(3, w1), 0).astype(np.float32)
+    F32 = O.Prec("f32")
+    k, v = runner.vm["prefill"](dev(prefix), dev(pm), params)
+    kr, vr = O.prefill(p, d, prefix, pm, F32)
+    _tol(k.numpy()[..., :valid, :], kr[..., :valid, :], "keys")
+    _tol(v.numpy()[..., :valid, :], vr[..., :valid, :], "values")
+    kd, vd = dev(kr), dev(vr)
+    got = runner.vm["denoise_step_kv"](kd, vd, dev(x), dev(te[:1]), dev(cos), dev(sin), dev(pm), params)
+    _tol(got.numpy(), O.denoise_step_kv(p, d, kr, vr, x, te[:1], cos, sin, pm, F32), "velocity")
+    loop = runner.vm["denoise_loop_kv"](kd, vd, dev(x), dev(te), dev(cos), dev(sin), dev(pm), params)
+    _tol(loop.numpy(), O.denoise_loop_kv(p, d, kr, vr, x, te, cos, sin, pm, F32), "loop")
+    runner.vm.set_graph(True)
+    chunk = [runner.vm["chunk"](dev(prefix), dev(pm), dev(x), dev(te), dev(cos), dev(sin), params).numpy()
+             for _ in range(2)]
+    _tol(chunk[0], loop.numpy(), "chunk")
+    np.testing.assert_array_equal(chunk[1], chunk[0])
