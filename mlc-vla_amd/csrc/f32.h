@@ -52,4 +52,21 @@ struct F32Op {
 };
 int f32_gemm_launch(const F32Op& a, hipStream_t st);
 
+// softmax(q . k + mask) . v over the prefix keys kp / vp [KV][Sp][hd] (additive mask [Sp] or null) and
+// the suffix rows ks / vs [Ts][s_ld] (kv head h at h hd): q [Tq][q_ld] -> out [Tq][o_ld], query head h
+// at h hd reading kv head h / (H / KV).  hd one of 16, 32, 64, 128, 256; 16-byte aligned rows.
+struct F32Attn {
+  const float* q;
+  int q_ld, Tq, H, KV, hd;
+  const float *kp, *vp;
+  int Sp;
+  const float* mask;
+  const float *ks, *vs;
+  int s_ld, Ts;
+  float* out;
+  int o_ld;
+  float* ws;  // f32_attn_ws_floats of the plan
+};
+int f32_attn_launch(const F32Attn& a, hipStream_t st);
+
 }  // namespace mlcv

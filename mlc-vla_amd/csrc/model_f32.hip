@@ -255,6 +255,7 @@ struct F32Model {
   // step
   float *x, *xn, *q, *k, *v, *attn, *o, *gu, *h, *cond, *tmp, *mods, *vout, *x32;
   float *scos, *ssin, *smask, *te, *xt;
+  float* aws = nullptr;  // split partials of the attention
 
   ~F32Model() {
     for (void* p : owned) (void)hipFree(p);
@@ -346,6 +347,28 @@ F32Op qkv_op(const F32Model& m, const F32Lin& q, const F32Lin& k, const F32Lin& 
   return a;
 }
 
+int fast_attn(const F32Model& m, const float* q, int rows, const float* kp, const float* vp, const float* mask,
+              const float* ks, const float* vs, int Ts, float* out, hipStream_t st) {
+  F32Attn a{};
+  a.q = q;
+  a.q_ld = a.o_ld = m.H * m.HD;
+  a.Tq = rows;
+  a.H = m.H;
+  a.KV = m.KV;
+  a.hd = m.HD;
+  a.kp = kp;
+  a.vp = vp;
+  a.Sp = m.P;
+  a.mask = mask;
+  a.ks = ks;
+  a.vs = vs;
+  a.s_ld = m.KV * m.HD;
+  a.Ts = Ts;
+  a.out = out;
+  a.ws = m.aws;
+  return f32_attn_launch(a, st);
+}
+
 // the time MLP and every modulation of `steps` time embeddings te [steps][W1] into mods
 // [steps][2 D + 1][3 W1]
 int f32_mods(F32Model& m, const float* te, int steps, hipStream_t st) {
@@ -379,7 +402,7 @@ int f32_velocity(F32Model& m, const float* keys, const float* values, const floa
     a.mod = mi;
     a.xn = m.xn;
     MLCV_TRY(f32_gemm_launch(a, st));
-    MLCV_TRY(attn(m.q, nq, m, keys + L * kvs, values + L * kvs, m.P, pmask, m.k, m.v, nkv, T, m.attn, T, st));
+    MLCV_TRY(fast_attn(m, m.q, T, keys + L * kvs, values + L * kvs, pmask, m.k, m.v, T, m.attn, st));
     a = lin_op(m.attn, nq, T, ly.o[1], FE_RES, m.x, W1);
     a.gate = mi + 2 * W1;
     MLCV_TRY(f32_gemm_launch(a, st));
@@ -414,7 +437,7 @@ int f32_prefix(F32Model& m, float* keys, float* values, hipStream_t st) {
     a.xn = m.pxn;
     MLCV_TRY(f32_gemm_launch(a, st));
     if (last) break;
-    MLCV_TRY(attn(m.pq, nq, m, kL, vL, P, m.mask, nullptr, nullptr, 0, 0, m.pattn, P, st));
+    MLCV_TRY(fast_attn(m, m.pq, P, kL, vL, m.mask, nullptr, nullptr, 0, m.pattn, st));
     MLCV_TRY(f32_gemm_launch(lin_op(m.pattn, nq, P, ly.o[0], FE_RES, m.px, W0), st));
     a = lin_op(m.px, W0, P, ly.gu[0], FE_GEGLU, m.ph, m.F0);
     a.F = m.F0;
@@ -501,6 +524,13 @@ int f32_create(const ::mlcv_config& cfg, F32Model** out) {
            {&r.scos, T * r.HD / 2}, {&r.ssin, T * r.HD / 2}, {&r.smask, P}, {&r.te, (size_t)r.S * r.W1},
            {&r.xt, T * r.A}})
     MLCV_TRY(r.alloc(p, n));
+  size_t aws = 0;
+  for (auto [rows, nk] : {std::pair<int, int>{r.P, r.P}, {r.T, r.P + r.T}}) {
+    int ns = 1, cps = 1;
+    f32_attn_plan(rows * (r.H / r.KV), r.KV, nk, &ns, &cps);
+    aws = std::max(aws, f32_attn_ws_floats(r.KV, rows * (r.H / r.KV), r.HD, ns));
+  }
+  MLCV_TRY(r.alloc(&r.aws, aws));
   // RoPE of the prefill's positions 0..P-1: radians = pos / theta^((2/hd) i) in float64
   std::vector<float> hc(P * r.HD / 2), hs(P * r.HD / 2);
   for (size_t p = 0; p < P; ++p)

@@ -35,6 +35,23 @@ inline size_t attn_ws_floats(int KV, int rows, int hd, int nsplit) {
   return nsplit > 1 ? (size_t)KV * nsplit * rpad * (hd + 2) : 0;
 }
 
+// ---- float32 attention (attn_f32.hip) ------------------------------------------------------
+constexpr int F32_ATTN_TARGET = 512;  // workgroups: two per CU
+// Key splits of `rows` query rows per kv head against nk keys: about two workgroups per CU, at least
+// two chunks per split (a split costs its partials and the combine launch), none empty.
+// *cps: chunks per split.
+inline void f32_attn_plan(int rows, int KV, int nk, int* nsplit, int* cps) {
+  const int rb = (rows + ATTN_ROWS - 1) / ATTN_ROWS * KV, chunks = (nk + ATTN_KCH - 1) / ATTN_KCH;
+  const int ns = std::max(1, std::min({F32_ATTN_TARGET / std::max(rb, 1), (chunks + 1) / 2, 64}));
+  *cps = std::max(1, (chunks + ns - 1) / ns);
+  *nsplit = std::max(1, (chunks + *cps - 1) / *cps);
+}
+// fp32 partials O [KV][nsplit][rpad][hd], then (m, l) [KV][nsplit][rpad][2]; none for one split
+inline size_t f32_attn_ws_floats(int KV, int rows, int hd, int nsplit) {
+  const size_t rpad = (size_t)((rows + ATTN_ROWS - 1) / ATTN_ROWS) * ATTN_ROWS;
+  return nsplit > 1 ? (size_t)KV * nsplit * rpad * (hd + 2) : 0;
+}
+
 // ---- skinny GEMM (gemm_skinny.hip) ------------------------------------------------------
 constexpr int SK_KC = 128;        // k per chunk
 constexpr int SK_MAX_SPLIT = 8;   // K slices at most

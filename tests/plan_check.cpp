@@ -62,6 +62,22 @@ static void check_attn() {
         }
 }
 
+static void check_f32_attn() {
+  for (int rows : {1, 16, 63, 64, 65, 400, 7744})
+    for (int KV : {1, 2, 8})
+      for (int nk : {1, 31, 32, 33, 64, 65, 100, 968, 1018, 16000}) {
+        int ns = -1, cps = -1;
+        f32_attn_plan(rows, KV, nk, &ns, &cps);
+        ++checked;
+        const int chunks = (nk + ATTN_KCH - 1) / ATTN_KCH;
+        CHECK(ns >= 1 && ns <= 64 && cps >= 1, "rows %d KV %d nk %d: %d x %d", rows, KV, nk, ns, cps);
+        CHECK((long)ns * cps >= chunks && (long)(ns - 1) * cps < chunks, "rows %d nk %d: %d x %d chunks of %d", rows, nk, ns, cps, chunks);
+        const size_t rpad = (size_t)((rows + ATTN_ROWS - 1) / ATTN_ROWS) * ATTN_ROWS, hd = 256;
+        const size_t end = (size_t)KV * ns * rpad * hd + 2 * ((((size_t)KV - 1) * ns + ns - 1) * rpad + rows);
+        CHECK(ns == 1 || end <= f32_attn_ws_floats(KV, rows, (int)hd, ns), "partials past the workspace");
+      }
+}
+
 static void check_skinny() {
   for (int ntiles : {1, 2, 3, 8, 16, 40, 64, 160, 256, 512, 1024})
     for (int K : {32, 96, 128, 129, 512, 1024, 2048, 4096, 16384})
@@ -156,6 +172,7 @@ static void check_tile() {
 
 int main() {
   check_attn();
+  check_f32_attn();
   check_skinny();
   check_modulations();
   check_tile();
