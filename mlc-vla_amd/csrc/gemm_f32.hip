@@ -69,20 +69,43 @@ __device__ __forceinline__ const float* w_row(const F32Op& a, const float* w0, i
   }
 }
 
+// What an epilogue reads for the quad n .. n + 3 of row m besides the product: FE_STORE u = bias;
+// FE_RES u = the old value, v = gate; FE_EULER u = the old value, v = bias; FE_QKV (q, k) u = cos, v = sin
+struct EpiIn {
+  f4 u, v;
+};
+template <int EPI>
+__device__ __forceinline__ EpiIn epi_in(const F32Op& a, const float* b, const float* out, int m, int n) {
+  EpiIn e{};
+  if constexpr (EPI == FE_STORE) {
+    if (b) e.u = ldg4(b + n);
+  } else if constexpr (EPI == FE_RES || EPI == FE_EULER) {
+    e.u = load_global(reinterpret_cast<const f4*>(out + (size_t)m * a.ldo + n));
+    const float* g = EPI == FE_RES ? a.gate : b;
+    if (g) e.v = ldg4(g + n);
+  } else if constexpr (EPI == FE_QKV) {
+    if (n < a.nq + a.nkv) {
+      const int nn = n < a.nq ? n : n - a.nq, d = 8 * ((nn >> 4) % (a.hd >> 4)) + (n & 7), half = a.hd >> 1;
+      e.u = ldg4(a.cos + (size_t)m * half + d);
+      e.v = ldg4(a.sin + (size_t)m * half + d);
+    }
+  }
+  return e;
+}
+
 // 4 consecutive outputs n .. n + 3 of row m, unpaired
 template <int EPI>
-__device__ __forceinline__ void epi_one(const F32Op& a, const float* b, float* out, int m, int n, f4 v) {
+__device__ __forceinline__ void epi_one(const F32Op& a, const float* b, float* out, int m, int n, f4 v,
+                                        const EpiIn& e) {
   if constexpr (EPI == FE_QKV) {  // v
     const int nn = n - a.nq - a.nkv, h = nn / a.hd, d = nn % a.hd;
     *reinterpret_cast<f4*>(a.vo + (size_t)m * a.kv_m + h * a.kv_h + d) = v;
     return;
   }
-  float* o = out + (size_t)m * a.ldo + n;
   if (EPI == FE_STORE || EPI == FE_EULER) {
     if (b) {
-      const f4 bv = ldg4(b + n);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = v[i] + bv[i];
+      for (int i = 0; i < 4; ++i) v[i] = v[i] + (EPI == FE_STORE ? e.u[i] : e.v[i]);
     }
   }
   if constexpr (EPI == FE_STORE) {
@@ -91,27 +114,25 @@ __device__ __forceinline__ void epi_one(const F32Op& a, const float* b, float* o
       for (int i = 0; i < 4; ++i) v[i] = v[i] / (1.0f + expf(-v[i]));
     }
   } else if constexpr (EPI == FE_RES) {
-    const f4 x = *reinterpret_cast<const f4*>(o);
-    const f4 g = a.gate ? ldg4(a.gate + n) : (f4){1.f, 1.f, 1.f, 1.f};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float y = v[i] * g[i];
-      v[i] = x[i] + y;
+      const float y = a.gate ? v[i] * e.v[i] : v[i];
+      v[i] = e.u[i] + y;
     }
   } else if constexpr (EPI == FE_EULER) {
-    const f4 x = *reinterpret_cast<const f4*>(o);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float y = a.dt * v[i];
-      v[i] = x[i] + y;
+      v[i] = e.u[i] + y;
     }
   }
-  *reinterpret_cast<f4*>(o) = v;
+  *reinterpret_cast<f4*>(out + (size_t)m * a.ldo + n) = v;
 }
 
-// outputs n .. n + 3 (the first 8 rows of a slab) and their partners n + 8 .. n + 11 of row m
+// outputs n .. n + 3 (the first 8 rows of a slab) and their partners n + 8 .. n + 11 of row m, of the
+// paired epilogues (FE_GEGLU, FE_QKV)
 template <int EPI>
-__device__ __forceinline__ void epi_pair(const F32Op& a, const float* b, float* out, int m, int n, f4 v, f4 vp) {
+__device__ __forceinline__ void epi_pair(const F32Op& a, float* out, int m, int n, f4 v, f4 vp, const EpiIn& e) {
   if constexpr (EPI == FE_GEGLU) {
     const float c = 0.7978845608028654f;  // sqrt(2 / pi)
     f4 h;
@@ -122,31 +143,28 @@ __device__ __forceinline__ void epi_pair(const F32Op& a, const float* b, float* 
       h[i] = g * vp[i];
     }
     *reinterpret_cast<f4*>(out + (size_t)m * a.ldo + 8 * (n >> 4) + (n & 7)) = h;
-  } else if constexpr (EPI == FE_QKV) {
+  } else {
     if (n >= a.nq + a.nkv) {
-      epi_one<EPI>(a, b, out, m, n, v);
-      epi_one<EPI>(a, b, out, m, n + 8, vp);
+      epi_one<EPI>(a, nullptr, out, m, n, v, e);
+      epi_one<EPI>(a, nullptr, out, m, n + 8, vp, e);
       return;
     }
     const bool k = n >= a.nq;
     const int nn = k ? n - a.nq : n, s = nn >> 4, spb = a.hd >> 4, h = s / spb, d = 8 * (s % spb) + (n & 7);
-    const int half = a.hd >> 1;
-    const f4 cs = ldg4(a.cos + (size_t)m * half + d), sn = ldg4(a.sin + (size_t)m * half + d);
     const float scale = k ? 1.0f : a.qscale;
     f4 o1, o2;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      o1[i] = (v[i] * cs[i] - vp[i] * sn[i]) * scale;
-      o2[i] = (vp[i] * cs[i] + v[i] * sn[i]) * scale;
+      o1[i] = (v[i] * e.u[i] - vp[i] * e.v[i]) * scale;
+      o2[i] = (vp[i] * e.u[i] + v[i] * e.v[i]) * scale;
     }
     float* o = k ? a.ko + (size_t)m * a.kv_m + h * a.kv_h + d : a.qo + (size_t)m * a.nq + h * a.hd + d;
     *reinterpret_cast<f4*>(o) = o1;
-    *reinterpret_cast<f4*>(o + half) = o2;
-  } else {
-    epi_one<EPI>(a, b, out, m, n, v);
-    if (n + 8 < a.N) epi_one<EPI>(a, b, out, m, n + 8, vp);
+    *reinterpret_cast<f4*>(o + (a.hd >> 1)) = o2;
   }
 }
+template <int EPI>
+constexpr bool epi_paired() { return EPI == FE_GEGLU || EPI == FE_QKV; }
 
 // ---- many rows ---------------------------------------------------------------------------
 constexpr int FT_BK = 32;  // k per stage: 128-byte rows in LDS, 8 pieces of 16 bytes
@@ -258,8 +276,14 @@ __global__ __launch_bounds__(256) void f32_tile_kernel(const F32Op a, int mtiles
         const int n = n0 + wn * (BN / 2) + nb * 32 + 8 * q + 4 * lh;
         if (n >= a.N) continue;
         const f16v& v = acc[nb][mb];
-        epi_pair<EPI>(a, a.b, a.out, m, n, (f4){v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]},
-                      (f4){v[4 * q + 4], v[4 * q + 5], v[4 * q + 6], v[4 * q + 7]});
+        const f4 v0 = {v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+        const f4 v1 = {v[4 * q + 4], v[4 * q + 5], v[4 * q + 6], v[4 * q + 7]};
+        if constexpr (epi_paired<EPI>()) {
+          epi_pair<EPI>(a, a.out, m, n, v0, v1, epi_in<EPI>(a, a.b, a.out, m, n));
+        } else {
+          epi_one<EPI>(a, a.b, a.out, m, n, v0, epi_in<EPI>(a, a.b, a.out, m, n));
+          if (n + 8 < a.N) epi_one<EPI>(a, a.b, a.out, m, n + 8, v1, epi_in<EPI>(a, a.b, a.out, m, n + 8));
+        }
       }
     }
 }
@@ -267,11 +291,15 @@ __global__ __launch_bounds__(256) void f32_tile_kernel(const F32Op a, int mtiles
 // ---- few rows ------------------------------------------------------------------------------
 constexpr int FS_NW = 8;  // waves: each takes every 8th block of 32 k
 
-// NORM: 0 none, 1 RMSNorm, 2 adaRMS of the rows, in the loader
+// NORM: 0 none, 1 RMSNorm, 2 adaRMS of the rows, in one pass over x: the product takes x (1 + scale),
+// the rows' sums of squares are added up on the way, and y = product / sqrt(mean(x^2) + eps) + shift . w.
+// A launch is a chain of memory latencies, so everything it reads goes out before the first wait: the
+// first blocks of the weights and of x, then what the epilogue reads.
 template <int MT, int NORM, int EPI>
 __global__ __launch_bounds__(64 * FS_NW) void f32_skinny_kernel(const F32Op a) {
   __shared__ f4 red[FS_NW * MT * 64];
-  __shared__ float den[16 * MT];
+  __shared__ float ssq[NORM != 0 ? FS_NW * MT * 16 : 1];  // sums of squares [wave][row]
+  __shared__ float shw[NORM == 2 ? FS_NW * 16 : 1];       // shift . w [wave][weight row]
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
   const int m0 = blockIdx.y * 16 * MT, K = a.K;
@@ -282,28 +310,10 @@ __global__ __launch_bounds__(64 * FS_NW) void f32_skinny_kernel(const F32Op a) {
     b = a.tab[blockIdx.z].b;
     out += blockIdx.z * a.tab_stride;
   }
-  if constexpr (NORM != 0) {
-    for (int row = w; row < 16 * MT; row += FS_NW) {
-      const float* xr = a.x + (size_t)min(m0 + row, a.M - 1) * a.ldx;
-      float ss = 0.f;
-      for (int k = 4 * lane; k < K; k += 256) {
-        const f4 v = ldg4(xr + k);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ss = ss + v[i] * v[i];
-      }
-      ss = wave_sum(ss);
-      if (lane == 0) den[row] = sqrtf(ss / (float)K + a.eps);
-    }
-    __syncthreads();
-  }
   const float* wr = w_row<EPI>(a, w0, min(16 * (int)blockIdx.x + r, a.N - 1));
   const float* xr[MT];
-  float dn[MT];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    xr[mt] = a.x + (size_t)min(m0 + 16 * mt + r, a.M - 1) * a.ldx;
-    if constexpr (NORM != 0) dn[mt] = den[16 * mt + r];
-  }
+  for (int mt = 0; mt < MT; ++mt) xr[mt] = a.x + (size_t)min(m0 + 16 * mt + r, a.M - 1) * a.ldx;
   struct Blk {
     f4 w[2], x[MT][2], sc[2], sh[2];
   };
@@ -330,42 +340,66 @@ __global__ __launch_bounds__(64 * FS_NW) void f32_skinny_kernel(const F32Op a) {
     }
   };
   f4 acc[MT];
+  float ss[MT], sw = 0.f;
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) acc[mt] = (f4){0.f, 0.f, 0.f, 0.f};
+  for (int mt = 0; mt < MT; ++mt) {
+    acc[mt] = (f4){0.f, 0.f, 0.f, 0.f};
+    ss[mt] = 0.f;
+  }
   auto mul = [&](const Blk& t) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i) {
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
         f4 x = t.x[mt][i];
         if constexpr (NORM != 0) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const float xn = x[e] / dn[mt];
-            const float y = xn * (1.0f + t.sc[i][e]);
-            x[e] = NORM == 2 ? y + t.sh[i][e] : y;
+            ss[mt] = fmaf(x[e], x[e], ss[mt]);
+            x[e] = x[e] * (1.0f + t.sc[i][e]);
           }
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[mt] = mfma_f32_16(t.w[i][e], x[e], acc[mt]);
       }
+      if constexpr (NORM == 2) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sw = fmaf(t.w[i][e], t.sh[i][e], sw);
+      }
+    }
   };
   const int nc = (K + 31) / 32;
   Blk t0, t1;
   int c = w;
   if (c < nc) load(c, t0);
-  while (c < nc) {  // the next block's loads go out before this one multiplies
-    if (c + FS_NW < nc) load(c + FS_NW, t1);
+  if (c + FS_NW < nc) load(c + FS_NW, t1);
+  // waves 0 .. MT - 1 write the m tiles: lane's rows n = 4 g .. + 3 of column m = r
+  const int m = m0 + 16 * w + r, n = 16 * blockIdx.x + 4 * g;
+  const bool mine = w < MT && m < a.M && n < a.N && !(epi_paired<EPI>() && g >= 2);
+  EpiIn ein{};
+  if (mine) ein = epi_in<EPI>(a, b, out, m, n);
+  while (c < nc) {  // two blocks in flight
     mul(t0);
+    if (c + 2 * FS_NW < nc) load(c + 2 * FS_NW, t0);
     c += FS_NW;
     if (c >= nc) break;
-    if (c + FS_NW < nc) load(c + FS_NW, t0);
     mul(t1);
+    if (c + 2 * FS_NW < nc) load(c + 2 * FS_NW, t1);
     c += FS_NW;
   }
-  // the waves' products, summed in wave order; lane holds rows n = 4 g .. + 3 of column m = r
+  // the waves' products, summed in wave order
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) red[(w * MT + mt) * 64 + lane] = acc[mt];
+  for (int mt = 0; mt < MT; ++mt) {
+    red[(w * MT + mt) * 64 + lane] = acc[mt];
+    if constexpr (NORM != 0) {
+      const float s = xor_sum_16_32(ss[mt]);
+      if (g == 0) ssq[(w * MT + mt) * 16 + r] = s;
+    }
+  }
+  if constexpr (NORM == 2) {
+    const float s = xor_sum_16_32(sw);
+    if (g == 0) shw[w * 16 + r] = s;
+  }
   __syncthreads();
   if (w >= MT) return;
   f4 v = red[w * 64 + lane];
@@ -375,14 +409,29 @@ __global__ __launch_bounds__(64 * FS_NW) void f32_skinny_kernel(const F32Op a) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = v[i] + u[i];
   }
-  const int m = m0 + 16 * w + r, n = 16 * blockIdx.x + 4 * g;
-  if constexpr (EPI == FE_GEGLU || EPI == FE_QKV) {
+  if constexpr (NORM != 0) {
+    float s = 0.f;
+#pragma unroll
+    for (int q = 0; q < FS_NW; ++q) s = s + ssq[(q * MT + w) * 16 + r];
+    const float den = sqrtf(s / (float)K + a.eps);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[i] = v[i] / den;
+      if constexpr (NORM == 2) {
+        float sh = 0.f;
+#pragma unroll
+        for (int q = 0; q < FS_NW; ++q) sh = sh + shw[q * 16 + 4 * g + i];
+        v[i] = v[i] + sh;
+      }
+    }
+  }
+  if constexpr (epi_paired<EPI>()) {
     f4 vp;
 #pragma unroll
     for (int i = 0; i < 4; ++i) vp[i] = __shfl_xor(v[i], 32);  // rows 8 on
-    if (g < 2 && m < a.M && n < a.N) epi_pair<EPI>(a, b, out, m, n, v, vp);
+    if (mine) epi_pair<EPI>(a, out, m, n, v, vp, ein);
   } else {
-    if (m < a.M && n < a.N) epi_one<EPI>(a, b, out, m, n, v);
+    if (mine) epi_one<EPI>(a, b, out, m, n, v, ein);
   }
 }
 
@@ -454,8 +503,7 @@ int f32_gemm_launch(const F32Op& in, hipStream_t st) {
   // 16-row slabs whose waves share out K
   const int bm = a.M > 64 && t128 >= 2 * cus ? 128 : a.M > 32 && t64 >= cus ? 64 : 0;
   int norm = a.nw ? 1 : a.mod ? 2 : 0;
-  // the norm in the loader: every workgroup reads its rows twice, cheaper than a launch for small x
-  const bool fuse = norm != 0 && bm == 0 && (long)std::min(a.M, 64) * a.K <= 65536 && !a.tab;
+  const bool fuse = bm == 0 && !a.tab;  // in the skinny kernel's one pass; a launch before the tiles
   if (norm != 0 && !fuse) {
     MLCV_REQUIRE(a.xn, "float32 linear: no room for the normalised rows");
     f32_rows_norm_kernel<<<a.M, 256, 0, st>>>(a.x, a.ldx, a.K, a.nw, a.mod, a.eps, a.xn);
