@@ -48,6 +48,8 @@ __global__ __launch_bounds__(256, 2) void f32_fa_kernel(const FaArgs p) {
   const int row = blockIdx.x * ATTN_ROWS + 16 * w + r, rowc = min(row, p.rows - 1);
   const int h = kvh * grp + rowc / a.Tq, t = rowc % a.Tq;
 
+  const float* kp = a.kv ? load_global(a.kv) + a.kv_off : a.kp;
+  const float* vp = a.kv ? load_global(a.kv + 1) + a.kv_off : a.vp;
   f4 kr[NI], vr[NI];
   float mr = 0.f;
   auto load = [&](int c) __attribute__((always_inline)) {
@@ -57,8 +59,8 @@ __global__ __launch_bounds__(256, 2) void f32_fa_kernel(const FaArgs p) {
       const int kj = min(c * ATTN_KCH + it / PPR, nk - 1), d = it % PPR * 4;  // past the keys: the last one
       const size_t pre = ((size_t)kvh * a.Sp + kj) * HD + d, suf = (size_t)(kj - a.Sp) * a.s_ld + kvh * HD + d;
       const bool in = kj < a.Sp;
-      kr[i] = load_global(reinterpret_cast<const f4*>(in ? a.kp + pre : a.ks + suf));
-      vr[i] = load_global(reinterpret_cast<const f4*>(in ? a.vp + pre : a.vs + suf));
+      kr[i] = load_global(reinterpret_cast<const f4*>(in ? kp + pre : a.ks + suf));
+      vr[i] = load_global(reinterpret_cast<const f4*>(in ? vp + pre : a.vs + suf));
     }
     if (tid < ATTN_KCH) {
       const int kj = c * ATTN_KCH + tid;

@@ -1358,10 +1358,11 @@ int mlcv_destroy(mlcv_ctx* ctx) {
 
 int mlcv_set_option(mlcv_ctx* ctx, int32_t key, int64_t value) {
   MLCV_REQUIRE(ctx, "null context");
-  if (ctx->f32) {  // the float32 model runs eager launches; the step-form options do not apply
+  if (ctx->f32) {  // the float32 model has one form of its step
     MLCV_REQUIRE(key == MLCV_OPT_USE_GRAPH || key == MLCV_OPT_HOIST_MODULATION || key == MLCV_OPT_MASK_SKIP ||
                      key == MLCV_OPT_STEP_GRAPH,
                  "this option is not built for float32 models");
+    if (key == MLCV_OPT_USE_GRAPH) f32_set_graph(*ctx->f32, value != 0);
     return 0;
   }
   Ctx& c = ctx->c;

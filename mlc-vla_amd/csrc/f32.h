@@ -59,6 +59,8 @@ struct F32Attn {
   const float* q;
   int q_ld, Tq, H, KV, hd;
   const float *kp, *vp;
+  const float* const* kv;  // or: kp = kv[0] + kv_off, vp = kv[1] + kv_off, read on the device (a
+  size_t kv_off;           // captured launch then serves any cache)
   int Sp;
   const float* mask;
   const float *ks, *vs;

@@ -372,6 +372,7 @@ int euler_init_launch(const float* x0, float* x32, _Float16* x16, int n, hipStre
 struct F32Model;
 int f32_create(const ::mlcv_config& cfg, F32Model** out);
 void f32_destroy(F32Model* m);
+void f32_set_graph(F32Model& m, bool on);
 int f32_bind(F32Model& m, const void* const* ptrs, int count);
 int f32_prefill(F32Model& m, const void* prefix_embs, const float* prefix_mask, float* keys, void* values,
                 hipStream_t st);

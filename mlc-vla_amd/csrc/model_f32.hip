@@ -245,6 +245,14 @@ struct F32Model {
   // the matrix-core kernels (gemm_f32.hip) take these widths and weight pointers; else the general ones
   bool shape_ok = false, fast = false;
   F32Tab* tab = nullptr;  // the 2 D + 1 modulations' weights and biases (device)
+  // the loop and the chunk as captured graphs over the model's own buffers (MLCV_OPT_USE_GRAPH): the
+  // inputs are staged into them and the caller's cache is reached through kvp, so a graph serves
+  // every call until the parameters are bound again
+  bool use_graph = true;
+  hipGraphExec_t g_loop = nullptr, g_chunk = nullptr;
+  hipStream_t cap = nullptr;
+  const float** kvp = nullptr;  // device: {keys, values} of the loop's call
+  int SB = 1;                   // steps whose modulations are made in one go
   std::vector<F32Layer> layers;
   F32Lin final_mod, ain, aout, tin, tout;
   std::vector<void*> owned;
@@ -260,6 +268,15 @@ struct F32Model {
   ~F32Model() {
     for (void* p : owned) (void)hipFree(p);
     if (tab) (void)hipFree(tab);
+    if (kvp) (void)hipFree(kvp);
+    drop_graphs();
+    if (cap) (void)hipStreamDestroy(cap);
+  }
+  void drop_graphs() {
+    for (hipGraphExec_t* g : {&g_loop, &g_chunk}) {
+      if (*g) (void)hipGraphExecDestroy(*g);
+      *g = nullptr;
+    }
   }
   int alloc(float** p, size_t n) {
     MLCV_HIP(hipMalloc(reinterpret_cast<void**>(p), std::max<size_t>(n, 1) * sizeof(float)));
@@ -347,8 +364,9 @@ F32Op qkv_op(const F32Model& m, const F32Lin& q, const F32Lin& k, const F32Lin& 
   return a;
 }
 
-int fast_attn(const F32Model& m, const float* q, int rows, const float* kp, const float* vp, const float* mask,
-              const float* ks, const float* vs, int Ts, float* out, hipStream_t st) {
+// kv_off: with kp null, the cache slices at m.kvp[0 / 1] + kv_off
+int fast_attn(const F32Model& m, const float* q, int rows, const float* kp, const float* vp, size_t kv_off,
+              const float* mask, const float* ks, const float* vs, int Ts, float* out, hipStream_t st) {
   F32Attn a{};
   a.q = q;
   a.q_ld = a.o_ld = m.H * m.HD;
@@ -358,6 +376,8 @@ int fast_attn(const F32Model& m, const float* q, int rows, const float* kp, cons
   a.hd = m.HD;
   a.kp = kp;
   a.vp = vp;
+  a.kv = kp ? nullptr : m.kvp;
+  a.kv_off = kv_off;
   a.Sp = m.P;
   a.mask = mask;
   a.ks = ks;
@@ -386,7 +406,7 @@ int f32_mods(F32Model& m, const float* te, int steps, hipStream_t st) {
   return f32_gemm_launch(a, st);
 }
 
-// one velocity evaluation of x_t with the modulations mods [2 D + 1][3 W1]: into v_out, or (x32
+// one velocity evaluation (keys null: the cache at m.kvp) of x_t with the modulations mods [2 D + 1][3 W1]: into v_out, or (x32
 // non-null) the Euler update x32 += dt * v
 int f32_velocity(F32Model& m, const float* keys, const float* values, const float* x_t, const float* mods,
                  const float* cs, const float* sn, const float* pmask, float* v_out, float* x32, float dt,
@@ -402,7 +422,7 @@ int f32_velocity(F32Model& m, const float* keys, const float* values, const floa
     a.mod = mi;
     a.xn = m.xn;
     MLCV_TRY(f32_gemm_launch(a, st));
-    MLCV_TRY(fast_attn(m, m.q, T, keys + L * kvs, values + L * kvs, pmask, m.k, m.v, T, m.attn, st));
+    MLCV_TRY(fast_attn(m, m.q, T, keys ? keys + L * kvs : nullptr, keys ? values + L * kvs : nullptr, L * kvs, pmask, m.k, m.v, T, m.attn, st));
     a = lin_op(m.attn, nq, T, ly.o[1], FE_RES, m.x, W1);
     a.gate = mi + 2 * W1;
     MLCV_TRY(f32_gemm_launch(a, st));
@@ -437,7 +457,7 @@ int f32_prefix(F32Model& m, float* keys, float* values, hipStream_t st) {
     a.xn = m.pxn;
     MLCV_TRY(f32_gemm_launch(a, st));
     if (last) break;
-    MLCV_TRY(fast_attn(m, m.pq, P, kL, vL, m.mask, nullptr, nullptr, 0, m.pattn, st));
+    MLCV_TRY(fast_attn(m, m.pq, P, kL, vL, 0, m.mask, nullptr, nullptr, 0, m.pattn, st));
     MLCV_TRY(f32_gemm_launch(lin_op(m.pattn, nq, P, ly.o[0], FE_RES, m.px, W0), st));
     a = lin_op(m.px, W0, P, ly.gu[0], FE_GEGLU, m.ph, m.F0);
     a.F = m.F0;
@@ -448,6 +468,50 @@ int f32_prefix(F32Model& m, float* keys, float* values, hipStream_t st) {
     MLCV_TRY(f32_gemm_launch(lin_op(m.ph, m.F0, P, ly.dn[0], FE_RES, m.px, W0), st));
   }
   return 0;
+}
+
+// the model's S Euler steps on x32 from the staged time embeddings, tables and mask
+int f32_steps(F32Model& m, const float* keys, const float* values, const float* pmask, hipStream_t st) {
+  const float dt = (float)(-1.0 / m.S);
+  const size_t modstep = (size_t)(2 * m.D + 1) * 3 * m.W1;
+  for (int i = 0; i < m.S; ++i) {
+    if (i % m.SB == 0) MLCV_TRY(f32_mods(m, m.te + (size_t)i * m.W1, std::min(m.SB, m.S - i), st));
+    MLCV_TRY(f32_velocity(m, keys, values, m.x32, m.mods + (i % m.SB) * modstep, m.scos, m.ssin, pmask, nullptr, m.x32,
+                          dt, st));
+  }
+  return 0;
+}
+
+// `body` on the caller's stream: as a graph captured on the model's own stream at its first use, or
+// directly (graphs off, or the caller is capturing)
+template <class F>
+int f32_run(F32Model& m, hipGraphExec_t& g, hipStream_t user, F&& body) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  MLCV_HIP(hipStreamIsCapturing(user, &cs));
+  if (!m.use_graph || cs != hipStreamCaptureStatusNone) return body(user);
+  if (!g) {
+    if (!m.cap) MLCV_HIP(hipStreamCreateWithFlags(&m.cap, hipStreamNonBlocking));
+    MLCV_HIP(hipStreamBeginCapture(m.cap, hipStreamCaptureModeThreadLocal));
+    const int r = body(m.cap);
+    hipGraph_t graph = nullptr;
+    const hipError_t e = hipStreamEndCapture(m.cap, &graph);
+    if (r != 0 || e != hipSuccess) {
+      if (e == hipSuccess && graph) (void)hipGraphDestroy(graph);
+      if (r != 0) return r;
+      MLCV_HIP(e);
+    }
+    const hipError_t ie = hipGraphInstantiate(&g, graph, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(graph);
+    if (ie != hipSuccess) g = nullptr;
+    MLCV_HIP(ie);
+  }
+  MLCV_HIP(hipGraphLaunch(g, user));
+  return 0;
+}
+
+__global__ void f32_set_kv_kernel(const float** kvp, const float* keys, const float* values) {
+  kvp[0] = keys;
+  kvp[1] = values;
 }
 
 // The general form of one velocity evaluation, for widths or pointers the matrix-core kernels do not
@@ -511,6 +575,8 @@ int f32_create(const ::mlcv_config& cfg, F32Model** out) {
                 m->F0 % 8 == 0 && m->W1 % 8 == 0 && m->F1 % 8 == 0 && m->A % 8 == 0;
   MLCV_REQUIRE(m->HD % 2 == 0 && m->H % m->KV == 0, "float32 model: head_dim even, heads a multiple of kv heads");
   MLCV_REQUIRE((size_t)(m->HD + m->P + m->T) * 4 <= 64 * 1024, "float32 model: prefix_len + suffix_len too large");
+  m->SB = std::min(m->S, 64);
+  const size_t SB = m->SB;
   const size_t P = m->P, T = m->T, nq = (size_t)m->H * m->HD, nkv = (size_t)m->KV * m->HD;
   const size_t kv = (size_t)m->D * nkv * P;
   F32Model& r = *m;
@@ -519,8 +585,8 @@ int f32_create(const ::mlcv_config& cfg, F32Model** out) {
            {&r.pattn, P * nq}, {&r.po, P * r.W0}, {&r.pgu, P * 2 * r.F0}, {&r.ph, P * r.F0},
            {&r.pcos, P * r.HD / 2}, {&r.psin, P * r.HD / 2}, {&r.mask, P}, {&r.ckeys, kv}, {&r.cvalues, kv},
            {&r.x, T * r.W1}, {&r.xn, T * r.W1}, {&r.q, T * nq}, {&r.k, T * nkv}, {&r.v, T * nkv},
-           {&r.attn, T * nq}, {&r.o, T * r.W1}, {&r.gu, T * 2 * r.F1}, {&r.h, T * r.F1}, {&r.cond, r.W1},
-           {&r.tmp, r.W1}, {&r.mods, (size_t)(2 * r.D + 1) * 3 * r.W1}, {&r.vout, T * r.A}, {&r.x32, T * r.A},
+           {&r.attn, T * nq}, {&r.o, T * r.W1}, {&r.gu, T * 2 * r.F1}, {&r.h, T * r.F1}, {&r.cond, SB * r.W1},
+           {&r.tmp, SB * r.W1}, {&r.mods, SB * (2 * r.D + 1) * 3 * r.W1}, {&r.vout, T * r.A}, {&r.x32, T * r.A},
            {&r.scos, T * r.HD / 2}, {&r.ssin, T * r.HD / 2}, {&r.smask, P}, {&r.te, (size_t)r.S * r.W1},
            {&r.xt, T * r.A}})
     MLCV_TRY(r.alloc(p, n));
@@ -531,6 +597,7 @@ int f32_create(const ::mlcv_config& cfg, F32Model** out) {
     aws = std::max(aws, f32_attn_ws_floats(r.KV, rows * (r.H / r.KV), r.HD, ns));
   }
   MLCV_TRY(r.alloc(&r.aws, aws));
+  MLCV_HIP(hipMalloc(reinterpret_cast<void**>(&r.kvp), 2 * sizeof(float*)));
   // RoPE of the prefill's positions 0..P-1: radians = pos / theta^((2/hd) i) in float64
   std::vector<float> hc(P * r.HD / 2), hs(P * r.HD / 2);
   for (size_t p = 0; p < P; ++p)
@@ -547,8 +614,14 @@ int f32_create(const ::mlcv_config& cfg, F32Model** out) {
 
 void f32_destroy(F32Model* m) { delete m; }
 
+void f32_set_graph(F32Model& m, bool on) {
+  m.use_graph = on;
+  m.drop_graphs();
+}
+
 int f32_bind(F32Model& m, const void* const* ptrs, int count) {
   m.bound = false;
+  m.drop_graphs();
   int idx = 0;
   auto f = [&]() { return reinterpret_cast<const float*>(ptrs[idx++]); };
   auto lin = [&](F32Lin& l, int N, int K, bool bias) {
@@ -607,8 +680,8 @@ int f32_prefill(F32Model& m, const void* prefix_embs, const float* prefix_mask, 
   const size_t kvs = (size_t)m.KV * P * m.HD;
   float* vals = reinterpret_cast<float*>(values);
   const float scale = 1.0f / std::sqrt((float)m.HD);
-  MLCV_HIP(hipMemcpyAsync(m.px, prefix_embs, (size_t)P * W0 * 4, hipMemcpyDeviceToDevice, st));
-  MLCV_HIP(hipMemcpyAsync(m.mask, prefix_mask, (size_t)P * 4, hipMemcpyDeviceToDevice, st));
+  const CopyJob in[] = {{prefix_embs, m.px, (size_t)P * W0 * 4}, {prefix_mask, m.mask, (size_t)P * 4}};
+  MLCV_TRY(copy_list_launch(in, 2, st));
   if (m.fast && f32_aligned({keys, values})) return f32_prefix(m, keys, vals, st);
   for (int L = 0; L < m.D; ++L) {
     const F32Layer& ly = m.layers[L];
@@ -649,30 +722,49 @@ int f32_step(F32Model& m, const float* keys, const void* values, const void* x_t
 int f32_loop(F32Model& m, const float* keys, const void* values, const float* x0, const void* time_embs,
              const float* cs, const float* sn, const float* prefix_mask, float* x_out, hipStream_t st) {
   MLCV_REQUIRE(m.bound, "parameters not bound");
-  const int n = m.T * m.A;
-  const float dt = (float)(-1.0 / m.S);
-  MLCV_HIP(hipMemcpyAsync(m.x32, x0, (size_t)n * 4, hipMemcpyDeviceToDevice, st));
+  const size_t n = (size_t)m.T * m.A, half = m.HD / 2;
   const float* vals = reinterpret_cast<const float*>(values);
   const float* te = reinterpret_cast<const float*>(time_embs);
-  const bool fast = m.fast && f32_aligned({keys, vals, te, cs, sn});
-  for (int i = 0; i < m.S; ++i) {
-    if (fast) {
-      MLCV_TRY(f32_mods(m, te + (size_t)i * m.W1, 1, st));
-      MLCV_TRY(f32_velocity(m, keys, vals, m.x32, m.mods, cs, sn, prefix_mask, nullptr, m.x32, dt, st));
-      continue;
-    }
-    MLCV_TRY(f32_step_general(m, keys, vals, m.x32, te + (size_t)i * m.W1, cs, sn, prefix_mask, m.vout, st));
-    f32_euler_kernel<<<ew_grid(n), 256, 0, st>>>(m.x32, m.vout, dt, n);
+  const CopyJob in[] = {{x0, m.x32, n * 4},
+                        {te, m.te, (size_t)m.S * m.W1 * 4},
+                        {cs, m.scos, m.T * half * 4},
+                        {sn, m.ssin, m.T * half * 4},
+                        {prefix_mask, m.smask, (size_t)m.P * 4}};
+  MLCV_TRY(copy_list_launch(in, 5, st));
+  if (m.fast && f32_aligned({keys, vals})) {
+    f32_set_kv_kernel<<<1, 1, 0, st>>>(m.kvp, keys, vals);
     MLCV_HIP(hipGetLastError());
+    MLCV_TRY(f32_run(m, m.g_loop, st, [&](hipStream_t s) { return f32_steps(m, nullptr, nullptr, m.smask, s); }));
+  } else {
+    const float dt = (float)(-1.0 / m.S);
+    for (int i = 0; i < m.S; ++i) {
+      MLCV_TRY(f32_step_general(m, keys, vals, m.x32, m.te + (size_t)i * m.W1, m.scos, m.ssin, m.smask, m.vout, st));
+      f32_euler_kernel<<<ew_grid(n), 256, 0, st>>>(m.x32, m.vout, dt, (int)n);
+      MLCV_HIP(hipGetLastError());
+    }
   }
-  MLCV_HIP(hipMemcpyAsync(x_out, m.x32, (size_t)n * 4, hipMemcpyDeviceToDevice, st));
-  return 0;
+  const CopyJob out{m.x32, x_out, n * 4};
+  return copy_list_launch(&out, 1, st);
 }
 
 int f32_chunk(F32Model& m, const void* prefix_embs, const float* prefix_mask, const float* x0, const void* time_embs,
               const float* cs, const float* sn, float* x_out, hipStream_t st) {
-  MLCV_TRY(f32_prefill(m, prefix_embs, prefix_mask, m.ckeys, m.cvalues, st));
-  return f32_loop(m, m.ckeys, m.cvalues, x0, time_embs, cs, sn, m.mask, x_out, st);
+  MLCV_REQUIRE(m.bound, "parameters not bound");
+  if (!m.fast) {
+    MLCV_TRY(f32_prefill(m, prefix_embs, prefix_mask, m.ckeys, m.cvalues, st));
+    return f32_loop(m, m.ckeys, m.cvalues, x0, time_embs, cs, sn, m.mask, x_out, st);
+  }
+  const size_t n = (size_t)m.T * m.A, half = m.HD / 2;
+  const CopyJob in[] = {{prefix_embs, m.px, (size_t)m.P * m.W0 * 4}, {prefix_mask, m.mask, (size_t)m.P * 4},
+                        {x0, m.x32, n * 4},                          {time_embs, m.te, (size_t)m.S * m.W1 * 4},
+                        {cs, m.scos, m.T * half * 4},                {sn, m.ssin, m.T * half * 4}};
+  MLCV_TRY(copy_list_launch(in, 6, st));
+  MLCV_TRY(f32_run(m, m.g_chunk, st, [&](hipStream_t s) {
+    MLCV_TRY(f32_prefix(m, m.ckeys, m.cvalues, s));
+    return f32_steps(m, m.ckeys, m.cvalues, m.mask, s);
+  }));
+  const CopyJob out{m.x32, x_out, n * 4};
+  return copy_list_launch(&out, 1, st);
 }
 
 }  // namespace mlcv

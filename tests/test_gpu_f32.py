@@ -75,6 +75,9 @@ def test_f32_model_vs_oracle(shape):
     loop = runner.vm["denoise_loop_kv"](kd, vd, dev(x), dev(te), dev(cos), dev(sin), dev(pm), params)
     _tol(loop.numpy(), O.denoise_loop_kv(p, d, kr, vr, x, te, cos, sin, pm, F32), "loop")
     runner.vm.set_graph(True)
+    for _ in range(3):  # captured once, replayed over other cache buffers
+        again = runner.vm["denoise_loop_kv"](dev(kr), dev(vr), dev(x), dev(te), dev(cos), dev(sin), dev(pm), params)
+        np.testing.assert_array_equal(again.numpy(), loop.numpy())
     chunk = [runner.vm["chunk"](dev(prefix), dev(pm), dev(x), dev(te), dev(cos), dev(sin), params).numpy()
              for _ in range(2)]
     _tol(chunk[0], loop.numpy(), "chunk")
