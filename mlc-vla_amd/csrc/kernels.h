@@ -236,6 +236,31 @@ int attn_launch(const AttnArgs& a, hipStream_t st);
 // (pinned host memory) and writes NaN rows
 int attn_fused_launch(const AttnArgs& a, unsigned* meet, unsigned polls, unsigned* err, hipStream_t st);
 
+// ---------------------------------------------------------------------------
+// fp16 linears over a few hundred rows (gemm_mid.hip): v = fp16(x . w^T), + bias in fp16, then
+// ---------------------------------------------------------------------------
+enum MidEpi : int {
+  ME_STORE = 0,     // y = v
+  ME_GELU = 1,      // y = fp16(gelu_tanh(v))
+  ME_RESIDUAL = 2,  // y = fp16(y + v)
+  ME_POS = 3,       // y = fp16(v + pos[m % npos])
+};
+struct MidArgs {
+  const _Float16* x;     // [M][ldx]
+  int ldx, M, K, N;
+  const _Float16* w[3];  // up to 3 matrices of rows [0, n1), [n1, n2), [n2, N), K halfs a row
+  const _Float16* b[3];  // their biases, or null
+  int n1, n2;
+  _Float16* y;           // [M][ldy]
+  int ldy, epi;
+  const _Float16* pos;   // ME_POS: [npos][N]
+  int npos;
+};
+bool mid_ok(const MidArgs& a);  // shapes and alignments the kernel takes
+int mid_gemm_launch(const MidArgs& a, hipStream_t st);
+// the weights of a later mid_gemm_launch of `a`, for `nblocks` prefetch workgroups of an earlier launch
+void mid_prefetch_add(const MidArgs& a, int nblocks, Prefetch& pf);
+
 // prefill helpers
 // tile: the output in the prefill GEMM's tile-major layout [ceil(rows / 16)][dim / 32][16][32]
 int rmsnorm_launch(const _Float16* x, const _Float16* w, _Float16* out, int rows, int dim, float eps,

@@ -100,6 +100,29 @@ inline size_t sk_mod_ws_floats(int NM, int W1, int mblocks) {
 // ---- prefill tile GEMM, 256-row tiles (gemm_tile.hip) -------------------------------------
 constexpr int TG_BM = 256, TG_BK = 64, TG_NXCD = 8;
 
+// ---- linears over a few hundred rows (gemm_mid.hip) ---------------------------------------
+enum MidTile : int { MID_64x96 = 0, MID_64x64 = 1, MID_32x64 = 2, MID_32x32 = 3 };
+// The tile with the least operand rows per CU, rounds of workgroups x (BM + BN): a CU takes its
+// tiles' rows out of the L2 at a fixed rate.  n tile j runs on XCD j % 8 with all its m tiles.  Ties go
+// to the larger tile.  *rows: that figure.
+inline int mid_plan(int M, int N, int cus, long* rows = nullptr) {
+  constexpr int BMS[4] = {64, 64, 32, 32}, BNS[4] = {96, 64, 64, 32};
+  int best = 0;
+  long least = 0;
+  for (int i = 0; i < 4; ++i) {
+    const long mt = (M + BMS[i] - 1) / BMS[i], nt = (N + BNS[i] - 1) / BNS[i];
+    const long xcd = (nt + TG_NXCD - 1) / TG_NXCD * mt, per = std::max(cus / TG_NXCD, 1);  // tiles, CUs per XCD
+    const long r = (xcd + per - 1) / per * (BMS[i] + BNS[i]);
+    if (i == 0 || r < least) {
+      best = i;
+      least = r;
+    }
+  }
+  if (rows) *rows = least;
+  return best;
+}
+
+// ---- the prefill tile GEMM's plan
 struct TilePlanIn {
   int M, N, K;
   int F;           // GeGLU: outputs (the gate rows, then F up rows)

@@ -97,6 +97,32 @@ static void check_skinny() {
         }
 }
 
+// The mid-size linears' tile: no other tile gives the busiest CU fewer operand rows, and ties go to the
+// larger one
+static void check_mid() {
+  const int bm[4] = {64, 64, 32, 32}, bn[4] = {96, 64, 64, 32};
+  for (int cus : {8, 64, 256, 304})
+    for (int M : {1, 32, 33, 64, 65, 100, 256, 457, 968, 1024})
+      for (int N : {4, 32, 36, 1024, 1152, 2048, 2560, 4304, 16384}) {
+        long rows = 0;
+        const int t = mid_plan(M, N, cus, &rows);
+        ++checked;
+        CHECK(t >= 0 && t < 4, "tile %d", t);
+        for (int i = 0; i < 4; ++i) {
+          // the busiest XCD's tiles, counted one by one
+          long most = 0;
+          for (int x = 0; x < 8; ++x) {
+            long n = 0;
+            for (int j = x; j * bn[i] < N; j += 8) n += (M + bm[i] - 1) / bm[i];
+            most = std::max(most, n);
+          }
+          const long per = std::max(cus / 8, 1), r = (most + per - 1) / per * (bm[i] + bn[i]);
+          CHECK(i == t ? r == rows : i < t ? r > rows : r >= rows, "M %d N %d: tile %d has %ld rows, %d has %ld", M, N,
+                t, rows, i, r);
+        }
+      }
+}
+
 // The modulation pieces of mlcv_bind_params on 64-row tiles (layer 0's two norms, then the other
 // NM - 2, 3 W1 rows each): the workspace mlcv_create allocates holds the partials of each piece.
 static void check_modulations() {
@@ -175,6 +201,7 @@ int main() {
   check_f32_attn();
   check_skinny();
   check_modulations();
+  check_mid();
   check_tile();
   std::printf("plans checked: %ld, failures: %d\n", checked, failures);
   return failures ? 1 : 0;

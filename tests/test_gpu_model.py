@@ -220,6 +220,50 @@ def test_vm_embed_image_vs_oracle(sig, tiny):
     np.testing.assert_array_equal(again, got[0])
 
 
+@pytest.mark.parametrize("sig,off", [
+    (dict(image_size=28, hidden_size=40, intermediate_size=40, num_attention_heads=8, projection_dim=36), 0),
+    (dict(image_size=70, hidden_size=72, intermediate_size=104, num_attention_heads=6, projection_dim=64), 0),
+    (dict(image_size=56, hidden_size=288, intermediate_size=328, num_attention_heads=2, projection_dim=100), 0),
+    (dict(image_size=42, hidden_size=256, intermediate_size=64, num_attention_heads=1, projection_dim=4), 0),
+    (dict(image_size=34, patch_size=2, hidden_size=80, intermediate_size=160, num_attention_heads=2, projection_dim=96), 0),
+    (dict(image_size=64, patch_size=2, hidden_size=96, intermediate_size=200, num_attention_heads=12, projection_dim=64), 0),
+    (dict(image_size=66, patch_size=2, hidden_size=96, intermediate_size=200, num_attention_heads=3, projection_dim=64), 0),
+    (dict(image_size=48, patch_size=2, hidden_size=544, intermediate_size=64, num_attention_heads=16, projection_dim=64), 0),
+    (dict(image_size=42, hidden_size=1600, intermediate_size=64, num_attention_heads=20, projection_dim=64), 0),
+    (dict(image_size=42, hidden_size=144, intermediate_size=200, num_attention_heads=2, projection_dim=64), 1),
+], ids=["hd5_4p", "hd12_25p", "hd144_16p", "hd256_9p", "hd40_289p", "hd8_1024p", "hd32_1089p", "hd34_576p", "ln1600", "off2bytes"])
+def test_vm_embed_image_shapes(sig, off, tiny):
+    """embed_image where its kernels have edges: head dims without 8-wide loads and up to 256, partial row
+    tiles and key chunks, widths with K and N tails, both LayerNorm register sizes, more than 1024 patches
+    (the long-M GEMM and an epilogue pass) and vectors 2 bytes off their alignment.  The tolerance of
+    test_vm_embed_image_vs_oracle."""
+    print(f"embed_image {sig} offset {off}", flush=True)
+    from mlc_vla import runtime
+    from mlc_vla.compile import compile_model
+    from mlc_vla.model.pi0 import Pi0Config, SiglipConfig
+    from oracle import siglip_oracle as S
+
+    sc = SiglipConfig(**{**dict(patch_size=14, num_hidden_layers=2), **sig})
+    ex, npar = compile_model(Pi0Config(**{**TINY_KWARGS, "siglip": sc}), "rocm", functions=["embed_image"])
+    vm = runtime.VirtualMachine(ex, tiny.runner.dev)
+    P = S.make_vision_params(sc, 11)
+
+    def dev(a):
+        if not off or a.ndim > 1:
+            return tiny.dev(a)
+        flat = tiny.dev(np.concatenate([np.zeros(1, np.float16), a]))
+        return runtime.Tensor(flat.torch[1:], "float16")
+
+    params = [dev(P[n]) for n, _ in npar]
+    for seed in (8, 9):
+        img = np.random.default_rng(seed).standard_normal((sc.image_size, sc.image_size, sc.num_channels)).astype(np.float16)
+        g = vm["embed_image"](tiny.dev(img[None]), params).numpy()[0].astype(np.float64)
+        ref = S.embed_image(P, sc, img, "f16")
+        assert g.shape == ref.shape and np.all(np.isfinite(g))
+        assert cosine(g, ref) >= 0.9999, cosine(g, ref)
+        assert max_abs(g, ref) <= 2e-2 * float(np.abs(ref).max()), (max_abs(g, ref), float(np.abs(ref).max()))
+
+
 def test_sample_vs_oracle_and_graph_loop(tiny):
     """sample (host loop) vs the oracle; sample_graph (device loop) vs sample (compare_loop)."""
     m = tiny
