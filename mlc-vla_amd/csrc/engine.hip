@@ -2400,11 +2400,41 @@ int mlcv_tile_linear(const void* x, int32_t M, int32_t K, const void* w, int32_t
   return tile_meet_failed(gerr, "mlcv_tile_linear");
 }
 
+// fp16 linears the mid-size kernel runs instead of the skinny one, which reads the weights once per 64
+// rows: from 65 rows on, K above 256.  Kernel times, skinny / mid, over 248 shapes of 65 to 1100 rows:
+// faster in all with K > 256 (100 x 2048 x 2048: 9.7 / 6.1 us, 457 x 2048 x 2560: 30.4 / 14.3,
+// 968 x 2048 x 2560: 46.5 / 26.2, 200 x 16384 x 2048: 95 / 37, 80 x 16384 x 1024: 29.0 / 26.6, the
+// closest), but 5.0 / 5.4 at 200 x 256 x 4096 and 4.9 / 8.7 at 968 x 64 x 2048, where the mid kernel's
+// start and its meeting outweigh its loop.
+static bool linear_mid(const void* x, int32_t M, int32_t K, const void* w, const void* bias, void* y, int32_t N,
+                       MidArgs* a) {
+  *a = MidArgs{};
+  a->x = reinterpret_cast<const _Float16*>(x);
+  a->ldx = K;
+  a->M = M;
+  a->K = K;
+  a->N = a->n1 = a->n2 = N;
+  for (int s = 0; s < 3; ++s) {
+    a->w[s] = reinterpret_cast<const _Float16*>(w);
+    a->b[s] = reinterpret_cast<const _Float16*>(bias);
+  }
+  a->y = reinterpret_cast<_Float16*>(y);
+  a->ldy = N;
+  a->epi = ME_STORE;
+  return w != nullptr && M > 64 && K > 256 && K % 32 == 0 && mid_ok(*a);
+}
+
 int mlcv_linear(const void* x, int32_t M, int32_t K, const void* w, const uint32_t* q_weight, const void* q_scale,
                 const void* bias, void* y, int32_t N, void* stream) {
   MLCV_REQUIRE(x && y && M > 0 && K > 0 && N > 0, "bad argument");
   MLCV_REQUIRE((w != nullptr) != (q_weight != nullptr && q_scale != nullptr), "pass either w or q_weight+q_scale");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  MidArgs mid;
+  if (linear_mid(x, M, K, w, bias, y, N, &mid)) {
+    MLCV_TRY(mid_gemm_launch(mid, st));
+    MLCV_HIP(hipStreamSynchronize(st));
+    return 0;
+  }
   SkSeg s{};
   s.w = reinterpret_cast<const _Float16*>(w);
   s.qw = q_weight;
@@ -2454,6 +2484,8 @@ int mlcv_linear_noalloc(const void* x, int32_t M, int32_t K, const void* w, cons
   MLCV_REQUIRE(sk_ws_floats(ntiles, mb, p, 64) <= NA_PART_FLOATS,
                "mlcv_linear_noalloc: the split-K partials exceed its scratch of " + std::to_string(NA_PART_FLOATS * 4) +
                    " bytes");
+  MidArgs mid;
+  if (linear_mid(x, M, K, w, bias, y, N, &mid)) return mid_gemm_launch(mid, st);
   char* base = nullptr;
   MLCV_TRY(noalloc_scratch(st, &base));
   SkSeg s{};

@@ -182,6 +182,50 @@ def test_linear_vs_oracle(m, k, n, q4):
     assert cosine(got, ref) > 0.99999
 
 
+# M, K, N, bias, offset (halfs, of y): around the row count and depth where the mid-size kernel takes over,
+# its four tiles, K tails of a stage, N of 4 mod 8, an output 8 bytes off its 16-byte alignment
+MID_SHAPES = [(64, 512, 64, True, 0), (65, 512, 64, True, 0), (65, 256, 64, True, 0), (65, 288, 4, False, 0),
+              (96, 544, 100, True, 0), (97, 2080, 1028, True, 0), (128, 1056, 4096, False, 0),
+              (200, 320, 32, True, 4), (256, 1152, 1152, True, 0), (256, 1152, 4304, True, 0), (457, 1024, 2560, True, 0),
+              (968, 512, 2052, False, 0), (1030, 16384, 16, True, 0)]
+
+
+@pytest.mark.parametrize("noalloc", [False, True], ids=["linear", "noalloc"])
+@pytest.mark.parametrize("m,k,n,bias,off", MID_SHAPES)
+def test_linear_many_rows(m, k, n, bias, off, noalloc):
+    """fp16 linears of more than 64 rows against the exact product, against the same rows in calls of 64
+    (the skinny kernel), and with a NaN and an infinity that stay in their rows."""
+    print(f"linear M={m} K={k} N={n} bias={bias} off={off} noalloc={noalloc}", flush=True)
+    rng = np.random.default_rng(m * 7 + k + n)
+    x = rng.standard_normal((m, k)).astype(np.float16)
+    w = (0.02 * rng.standard_normal((n, k))).astype(np.float16)
+    b = (0.02 * rng.standard_normal(n)).astype(np.float16)
+    x[3, k - 1], x[m - 1, 0] = np.inf, np.nan
+    xd, wd, bd = _dev(x), _dev(w), _dev(b)
+    fn = "mlcv_linear_noalloc" if noalloc else "mlcv_linear"
+    buf = torch.full((off + m * n + 8,), 7.0, dtype=torch.float16, device="cuda")
+    small = torch.empty((m, n), dtype=torch.float16, device="cuda")
+    N.call(fn, _p(xd), m, k, _p(wd), None, None, _p(bd) if bias else None, _p(buf[off:]), n, _st())
+    for r in range(0, m, 64):
+        N.call(fn, _p(xd[r:]), min(64, m - r), k, _p(wd), None, None, _p(bd) if bias else None, _p(small[r:]), n, _st())
+    flat = _host(buf)
+    assert np.all(flat[:off] == 7) and np.all(flat[off + m * n:] == 7)
+    got, ref = flat[off:off + m * n].reshape(m, n).astype(np.float64), _host(small).astype(np.float64)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(ref))
+    rows = [r for r in range(m) if r not in (3, m - 1)]
+    assert np.all(np.isfinite(got[rows])) and not np.any(np.isfinite(got[3])) and np.all(np.isnan(got[m - 1]))
+    got, ref, xr = got[rows], ref[rows], x[rows].astype(np.float64)
+    exact = xr @ w.astype(np.float64).T
+    # the fp32 sum: at most K / 16 + 32 sequential roundings (2^-24 each) of partial sums no larger than
+    # the sum of magnitudes; one rounding to fp16, one of the bias add (half an ulp each)
+    acc = (k / 16 + 32) * 2.0**-24 * (np.abs(xr) @ np.abs(w.astype(np.float64)).T)
+    full = exact + (b.astype(np.float64) if bias else 0.0)
+    bound = acc + 0.5 * _ulp16(np.abs(exact) + acc) + (0.5 * _ulp16(np.abs(full) + acc + _ulp16(exact)) if bias else 0.0)
+    assert np.all(np.abs(got - full) <= bound), float((np.abs(got - full) / bound).max())
+    assert np.all(np.abs(got - ref) <= 2 * bound), float((np.abs(got - ref) / bound).max())
+
+
 def _attn_case(tq, h, kv, hd, sp, ts, valid, k_f32, seed):
     rng = np.random.default_rng(seed)
     s = 1.0 / np.sqrt(hd)
