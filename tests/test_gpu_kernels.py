@@ -63,6 +63,37 @@ def test_q4_quantize_bitexact(n, k):
     np.testing.assert_array_equal(_host(qs).view(np.uint16), qs_ref.view(np.uint16))
 
 
+@pytest.mark.parametrize("n,k,off", [(1, 32, 1), (33, 992, 3), (32, 1024, 0), (129, 2048, 1)])
+def test_q4_quantize_ranges(n, k, off):
+    """Every magnitude of fp16 (subnormal groups, the largest values), groups of infinities, addresses of halfs."""
+    print(f"q4 quantize ranges N={n} K={k} off={off}", flush=True)
+    rng = np.random.default_rng(n * k)
+    scale = np.exp2(rng.uniform(-26, 15, size=(n, k // 32, 1)))
+    w = np.clip(rng.standard_normal((n, k // 32, 32)) * scale, -65504, 65504).astype(np.float16).reshape(n, k)
+    qw_ref, qs_ref = Q.quantize(w)
+    if n > 1:  # a group with infinities: scale inf, 7 (zero) for finite weights, 0 for the others; NaN counts as 0
+        w[1, :4] = [np.inf, -np.inf, np.nan, 1.0]
+        w[1, 4:32] = 0.0
+        qw_ref[1, :4] = [0x77777000, 0x77777777, 0x77777777, 0x77777777]
+        qs_ref[1, 0] = np.inf
+    buf = torch.zeros(n * k + off, dtype=torch.float16, device="cuda")
+    wd = buf[off:].view(n, k)
+    wd.copy_(_dev(w))
+    qw = torch.zeros((n, k // 8), dtype=torch.int32, device="cuda")
+    qs = torch.zeros((n, k // 32), dtype=torch.float16, device="cuda")
+    N.call("mlcv_q4_quantize", _p(wd), _p(qw), _p(qs), n, k, _st())
+    np.testing.assert_array_equal(_host(qw, np.uint32), qw_ref)
+    np.testing.assert_array_equal(_host(qs).view(np.uint16), qs_ref.view(np.uint16))
+    out = torch.zeros(n * k + off, dtype=torch.float16, device="cuda")
+    N.call("mlcv_q4_dequantize", _p(qw), _p(qs), _p(out[off:]), n, k, _st())
+    got, ref = _host(out[off:]).reshape(n, k), Q.dequantize(qw_ref, qs_ref)
+    keep = np.ones((n, k), bool)
+    if n > 1:
+        keep[1, :32] = False
+    np.testing.assert_array_equal(got.view(np.uint16)[keep], ref.view(np.uint16)[keep])
+    assert not _host(out[:off]).any()
+
+
 @pytest.mark.parametrize("n,k", [(7, 32), (3072, 1024), (64, 4096)])
 def test_q4_dequant_bitexact(n, k):
     print(f"q4 dequant N={n} K={k}", flush=True)
