@@ -2424,6 +2424,26 @@ static bool linear_mid(const void* x, int32_t M, int32_t K, const void* w, const
   return w != nullptr && M > 64 && K > 256 && K % 32 == 0 && mid_ok(*a);
 }
 
+// Linears that lin_rows_kernel runs instead of the skinny kernel: one round of workgroups, and rows x K up
+// to where its x reads (every workgroup's own, straight from the L2) outweigh the skinny kernel's staging
+// barriers and the meeting of its K slices.  From 4096 outputs on the skinny kernel's own workgroups read as
+// much of x, so the line lies higher; fp16 weights add four times the bytes of q4 to the same path, so there it
+// lies lower.  Skinny / lin_rows, us (q4; fp16), the 363 shapes measured inside are 1.01 to 4.2 times as fast:
+//   inside:  1 x 1024 x 1024  6.8 / 3.8; 6.6 / 4.2    50 x 1024 x 8192  8.8 / 6.9; 10.0 / 7.5
+//   near it: 64 x 512 x 512   5.1 / 5.0; 4.9 / 5.1    64 x 1024 x 4096  7.4 / 7.2; 7.2 / 7.6
+//   past it: 32 x 2048 x 512  6.5 / 7.6; 6.8 / 8.8    64 x 1024 x 16384 10.5 / 12.2; 12.6 / 15.1
+//            8 x 4096 x 512   8.3 / 8.9; -            968 x 256 x 1024  4.8 / 5.1; 4.5 / 5.4
+static bool linear_rows(const void* x, int32_t M, int32_t K, const void* w, const uint32_t* q_weight,
+                        const void* q_scale, const void* bias, void* y, int32_t N, LinRows* a) {
+  *a = LinRows{reinterpret_cast<const _Float16*>(x), M, K, N, reinterpret_cast<const _Float16*>(w), q_weight,
+               reinterpret_cast<const _Float16*>(q_scale), reinterpret_cast<const _Float16*>(bias),
+               reinterpret_cast<_Float16*>(y)};
+  const bool q4 = q_weight != nullptr, wide = N >= 4096 && M <= 64;
+  const long rk = (long)std::min(M, 64) * K, most = wide ? (q4 ? 65536 : 49152) : (q4 ? 32768 : 24576);
+  return rk <= most && K <= (N >= 1024 ? 2048 : 1024) &&
+         (long)((N + 31L) / 32) * ((M + 63L) / 64) <= std::max(device_cus(), 1) && lin_rows_ok(*a);
+}
+
 int mlcv_linear(const void* x, int32_t M, int32_t K, const void* w, const uint32_t* q_weight, const void* q_scale,
                 const void* bias, void* y, int32_t N, void* stream) {
   MLCV_REQUIRE(x && y && M > 0 && K > 0 && N > 0, "bad argument");
@@ -2432,6 +2452,12 @@ int mlcv_linear(const void* x, int32_t M, int32_t K, const void* w, const uint32
   MidArgs mid;
   if (linear_mid(x, M, K, w, bias, y, N, &mid)) {
     MLCV_TRY(mid_gemm_launch(mid, st));
+    MLCV_HIP(hipStreamSynchronize(st));
+    return 0;
+  }
+  LinRows lr;
+  if (linear_rows(x, M, K, w, q_weight, q_scale, bias, y, N, &lr)) {
+    MLCV_TRY(lin_rows_launch(lr, st));
     MLCV_HIP(hipStreamSynchronize(st));
     return 0;
   }
@@ -2486,6 +2512,8 @@ int mlcv_linear_noalloc(const void* x, int32_t M, int32_t K, const void* w, cons
                    " bytes");
   MidArgs mid;
   if (linear_mid(x, M, K, w, bias, y, N, &mid)) return mid_gemm_launch(mid, st);
+  LinRows lr;
+  if (linear_rows(x, M, K, w, q_weight, q_scale, bias, y, N, &lr)) return lin_rows_launch(lr, st);
   char* base = nullptr;
   MLCV_TRY(noalloc_scratch(st, &base));
   SkSeg s{};

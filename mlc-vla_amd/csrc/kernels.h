@@ -260,6 +260,17 @@ bool mid_ok(const MidArgs& a);  // shapes and alignments the kernel takes
 int mid_gemm_launch(const MidArgs& a, hipStream_t st);
 // the weights of a later mid_gemm_launch of `a`, for `nblocks` prefetch workgroups of an earlier launch
 void mid_prefetch_add(const MidArgs& a, int nblocks, Prefetch& pf);
+// y [M][N] = fp16(x [M][K] . w^T) [+ b], w [N][K] fp16 or q4f16_1 words and scales
+struct LinRows {
+  const _Float16* x;
+  int M, K, N;
+  const _Float16* w;   // or null
+  const uint32_t* qw;  // or null
+  const _Float16 *qs, *b;
+  _Float16* y;
+};
+bool lin_rows_ok(const LinRows& a);
+int lin_rows_launch(const LinRows& a, hipStream_t st);
 
 // prefill helpers
 // tile: the output in the prefill GEMM's tile-major layout [ceil(rows / 16)][dim / 32][16][32]

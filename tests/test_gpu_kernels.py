@@ -225,7 +225,7 @@ MID_SHAPES = [(64, 512, 64, True, 0), (65, 512, 64, True, 0), (65, 256, 64, True
 @pytest.mark.parametrize("m,k,n,bias,off", MID_SHAPES)
 def test_linear_many_rows(m, k, n, bias, off, noalloc):
     """fp16 linears of more than 64 rows against the exact product, against the same rows in calls of 64
-    (the skinny kernel), and with a NaN and an infinity that stay in their rows."""
+    (other kernels), and with a NaN and an infinity that stay in their rows."""
     print(f"linear M={m} K={k} N={n} bias={bias} off={off} noalloc={noalloc}", flush=True)
     rng = np.random.default_rng(m * 7 + k + n)
     x = rng.standard_normal((m, k)).astype(np.float16)
@@ -255,6 +255,54 @@ def test_linear_many_rows(m, k, n, bias, off, noalloc):
     bound = acc + 0.5 * _ulp16(np.abs(exact) + acc) + (0.5 * _ulp16(np.abs(full) + acc + _ulp16(exact)) if bias else 0.0)
     assert np.all(np.abs(got - full) <= bound), float((np.abs(got - full) / bound).max())
     assert np.all(np.abs(got - ref) <= 2 * bound), float((np.abs(got - ref) / bound).max())
+
+
+# M, K, N, bias, offset (halfs, of y): both sides of the row counts, depths and widths where the few-row kernel
+# takes over, one to 16 chunks a wave, half a chunk at the end, a wave without a chunk, N of 4 mod 8
+ROWS_SHAPES = [(1, 32, 4, True, 0), (1, 4096, 1028, True, 4), (4, 4128, 64, False, 0), (32, 2048, 36, True, 0),
+               (32, 2080, 64, True, 0), (33, 512, 4092, True, 0), (33, 544, 100, False, 4), (50, 1024, 8192, False, 0),
+               (64, 1024, 4096, True, 0), (64, 1056, 32, True, 0), (65, 96, 16384, True, 0), (127, 224, 448, True, 0),
+               (207, 288, 608, False, 0), (968, 512, 256, True, 0), (1000, 64, 1024, True, 0)]
+
+
+@pytest.mark.parametrize("q4", [False, True], ids=["f16", "q4"])
+@pytest.mark.parametrize("m,k,n,bias,off", ROWS_SHAPES)
+def test_linear_few_rows(m, k, n, bias, off, q4):
+    """Linears of few rows or short K through both entry points: the same bits, within the exact product's
+    bound, nothing written past the output, a NaN and an infinity that stay in their rows."""
+    print(f"linear M={m} K={k} N={n} bias={bias} off={off} q4={q4}", flush=True)
+    rng = np.random.default_rng(m * 7 + k + n)
+    x = rng.standard_normal((m, k)).astype(np.float16)
+    w = (0.02 * rng.standard_normal((n, k))).astype(np.float16)
+    b = (0.02 * rng.standard_normal(n)).astype(np.float16)
+    if m > 3:
+        x[3, k - 1], x[m - 1, 0] = np.inf, np.nan
+    args = (_dev(w), None, None)
+    if q4:
+        qw, qs = Q.quantize(w)
+        w = Q.dequantize(qw, qs)
+        args = (None, _dev(qw), _dev(qs))
+    xd, bd = _dev(x), _dev(b)
+    outs = []
+    for fn in ("mlcv_linear", "mlcv_linear_noalloc"):
+        buf = torch.full((off + m * n + 8,), 7.0, dtype=torch.float16, device="cuda")
+        N.call(fn, _p(xd), m, k, *(a if a is None else _p(a) for a in args), _p(bd) if bias else None, _p(buf[off:]), n,
+               _st())
+        flat = _host(buf)
+        assert np.all(flat[:off] == 7) and np.all(flat[off + m * n:] == 7)
+        outs.append(flat[off:off + m * n].reshape(m, n))
+    np.testing.assert_array_equal(outs[0].view(np.uint16), outs[1].view(np.uint16))
+    got = outs[0].astype(np.float64)
+    rows = [r for r in range(m) if m <= 3 or r not in (3, m - 1)]
+    if m > 3:
+        assert not np.any(np.isfinite(got[3])) and np.all(np.isnan(got[m - 1]))
+    got, xr = got[rows], x[rows].astype(np.float64)
+    exact = xr @ w.astype(np.float64).T
+    # as for many rows: at most K / 16 + 32 sequential roundings of the fp32 sum, one to fp16, one of the bias add
+    acc = (k / 16 + 32) * 2.0**-24 * (np.abs(xr) @ np.abs(w.astype(np.float64)).T)
+    full = exact + (b.astype(np.float64) if bias else 0.0)
+    bound = acc + 0.5 * _ulp16(np.abs(exact) + acc) + (0.5 * _ulp16(np.abs(full) + acc + _ulp16(exact)) if bias else 0.0)
+    assert np.all(np.abs(got - full) <= bound), float((np.abs(got - full) / bound).max())
 
 
 def _attn_case(tq, h, kv, hd, sp, ts, valid, k_f32, seed):
