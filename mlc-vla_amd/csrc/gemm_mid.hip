@@ -57,6 +57,11 @@ __global__ __launch_bounds__(64 * NW) void mid_gemm_kernel(const MidArgs a, int 
   const int l32 = lane & 31, lh = lane >> 5;
   // n tile j runs on XCD j % 8 (workgroups are dealt to the XCDs round-robin by id), all its m tiles:
   // a weight tile is fetched into one L2, and an earlier launch can have it fetched there
+  const int tiles = (ntiles + 7) / 8 * 8 * mtiles;
+  if ((int)blockIdx.x >= tiles) {
+    prefetch_run(a.pf, blockIdx.x, tiles);
+    return;
+  }
   const int j8 = blockIdx.x >> 3, tn = (blockIdx.x & 7) + 8 * (j8 / mtiles);
   if (tn >= ntiles) return;
   const int m0 = (j8 % mtiles) * BM, n0 = tn * BN;
@@ -194,7 +199,7 @@ __global__ __launch_bounds__(64 * NW) void mid_gemm_kernel(const MidArgs a, int 
 template <int BM, int BN, int NW, int NST>
 int launch(const MidArgs& a, hipStream_t st) {
   const int mt = (a.M + BM - 1) / BM, nt = (a.N + BN - 1) / BN;
-  const unsigned blocks = (unsigned)((nt + 7) / 8 * 8 * mt);
+  const unsigned blocks = (unsigned)((nt + 7) / 8 * 8 * mt + (a.pf.nreg > 0 ? a.pf.nblocks : 0));
   switch (a.epi) {
     case ME_STORE: mid_gemm_kernel<BM, BN, NW, NST, ME_STORE><<<blocks, 64 * NW, 0, st>>>(a, mt, nt); break;
     case ME_GELU: mid_gemm_kernel<BM, BN, NW, NST, ME_GELU><<<blocks, 64 * NW, 0, st>>>(a, mt, nt); break;
@@ -353,6 +358,13 @@ bool mid_ok(const MidArgs& a) {
          (a.n1 % 8 == 0 || a.n1 >= a.N) && (a.n2 % 8 == 0 || a.n2 >= a.N) && (p & 15) == 0 && (p8 & 7) == 0 &&
          (size_t)((a.N + 31) / 32 + 7) * ((a.M + 31) / 32) < (1u << 23) &&  // the grid
          (size_t)a.ldx * 256 < (1u << 30) && (size_t)a.K * 16 < (1u << 30);
+}
+
+int mid_spare(const MidArgs& a) {
+  constexpr int BMS[4] = {64, 64, 32, 32}, BNS[4] = {96, 64, 64, 32};  // MidTile
+  const int cus = std::max(device_cus(), 1), plan = mid_plan(a.M, a.N, cus);
+  const long mt = (a.M + BMS[plan] - 1) / BMS[plan], nt = (a.N + BNS[plan] - 1) / BNS[plan];
+  return (int)std::max(0L, cus - (nt + TG_NXCD - 1) / TG_NXCD * TG_NXCD * mt);
 }
 
 void mid_prefetch_add(const MidArgs& a, int nblocks, Prefetch& pf) {

@@ -255,7 +255,9 @@ struct MidArgs {
   int ldy, epi;
   const _Float16* pos;   // ME_POS: [npos][N]
   int npos;
+  Prefetch pf;           // prefetch workgroups appended to the grid (on CUs that the tiles leave idle)
 };
+int mid_spare(const MidArgs& a);  // CUs that its tiles leave idle
 bool mid_ok(const MidArgs& a);  // shapes and alignments the kernel takes
 int mid_gemm_launch(const MidArgs& a, hipStream_t st);
 // the weights of a later mid_gemm_launch of `a`, for `nblocks` prefetch workgroups of an earlier launch

@@ -42,8 +42,11 @@ __global__ void pad_cols_kernel(const _Float16* __restrict__ w, int k, int kp, _
 
 // Prefetch workgroups beside a LayerNorm's rows and beside an attention's tiles: the whole tower (27
 // layers of width 1152) takes 1754 us without either, 1720 with 128 beside the attention alone, 1743 with
-// 256 beside the LayerNorms alone, 1714 with both, 1718 with 512 each.
+// 256 beside the LayerNorms alone, 1714 with both, 1718 with 512 each.  With the LayerNorms' share on the
+// CUs that fc1 and fc2 leave idle instead (at least MID_PF_MIN of them): 1588; 8 layers of 4 / 64 / 196
+// patches 368 / 394 / 505 -> 328 / 365 / 474.
 constexpr int LN_PF = 256, ATTN_PF = 128;
+constexpr int MID_PF_MIN = 32;
 
 // Rows up to which a linear runs on gemm_mid.hip's small tiles, else on the long-M GEMM with an epilogue
 // pass.  4 layers of width 1152, us, without / with the small tiles: 256 patches 444 / 268, 1024 patches
@@ -499,12 +502,20 @@ int embed_image_enqueue(const VisionCfg& v, const _Float16* const* prm, const _F
   };
   // The weights of a linear come from HBM (a tower of 0.8 GB passes through the caches once per image),
   // which its own loads would wait out stage by stage: spare workgroups of the LayerNorm and attention
-  // launches before it, which are chains of latencies themselves, have them fetched.
+  // launches before it, which are chains of latencies themselves, have them fetched,
   auto prefetch = [&](std::initializer_list<const MidArgs*> ls, int nblocks) {
     Prefetch pf{};
     if (np <= MID_MAX_ROWS)
       for (const MidArgs* g : ls) mid_prefetch_add(*g, nblocks, pf);
     return pf;
+  };
+  // or, better, those beside an earlier linear, on the CUs that its own tiles leave idle (64 of 256 at fc1 and
+  // fc2 of 256 patches): `next`'s weights beside `g`.
+  auto beside = [&](MidArgs& g, const MidArgs& next) {
+    const int spare = np <= MID_MAX_ROWS && mid_ok(g) ? mid_spare(g) : 0;
+    if (spare < MID_PF_MIN) return false;
+    g.pf = prefetch({&next}, spare);
+    return g.pf.nreg > 0;
   };
 
   // patch embedding (+ bias) + position embedding
@@ -513,22 +524,30 @@ int embed_image_enqueue(const VisionCfg& v, const _Float16* const* prm, const _F
   MLCV_HIP(hipGetLastError());
   const _Float16* wp[1] = {wpad};
   MLCV_TRY(linear(args(patches, wp, prm + 1, 1, H, kp, x, ME_POS)));
+  const _Float16* const* tail = prm + 3 + 16 * v.layers;  // post LN w, b; projector w, b
+  const MidArgs ap = args(hn, tail + 2, tail + 3, 1, v.proj, H, out, ME_STORE);
+  bool ahead = false;  // the next linear after a LayerNorm has its weights on the way
   for (int L = 0; L < v.layers; ++L) {
     const _Float16* const* lp = prm + 3 + 16 * L;  // q w,b  k w,b  v w,b  o w,b  fc1 w,b  fc2 w,b  ln1 w,b  ln2 w,b
     const _Float16 *qw[3] = {lp[0], lp[2], lp[4]}, *qb[3] = {lp[1], lp[3], lp[5]};
-    const MidArgs aq = args(hn, qw, qb, 3, 3 * H, H, qkv, ME_STORE), ao = args(ctx, lp + 6, lp + 7, 1, H, H, x, ME_RESIDUAL),
-                  a1 = args(hn, lp + 8, lp + 9, 1, v.inter, H, u, ME_GELU), a2 = args(u, lp + 10, lp + 11, 1, H, v.inter, x, ME_RESIDUAL);
-    MLCV_TRY(layernorm(x, lp[12], lp[13], np, H, v.eps, hn, prefetch({&aq}, LN_PF), st));
+    const MidArgs aq = args(hn, qw, qb, 3, 3 * H, H, qkv, ME_STORE), ao = args(ctx, lp + 6, lp + 7, 1, H, H, x, ME_RESIDUAL);
+    MidArgs a1 = args(hn, lp + 8, lp + 9, 1, v.inter, H, u, ME_GELU), a2 = args(u, lp + 10, lp + 11, 1, H, v.inter, x, ME_RESIDUAL);
+    const bool ahead2 = beside(a1, a2);
+    MLCV_TRY(layernorm(x, lp[12], lp[13], np, H, v.eps, hn, ahead ? Prefetch{} : prefetch({&aq}, LN_PF), st));
     MLCV_TRY(linear(aq));
     MLCV_TRY(vis_attn(qkv, np, v.heads, hd, ctx, prefetch({&ao, &a1}, ATTN_PF), st));
     MLCV_TRY(linear(ao));
-    MLCV_TRY(layernorm(x, lp[14], lp[15], np, H, v.eps, hn, prefetch({&a2}, LN_PF), st));
+    MLCV_TRY(layernorm(x, lp[14], lp[15], np, H, v.eps, hn, ahead2 ? Prefetch{} : prefetch({&a2}, LN_PF), st));
     MLCV_TRY(linear(a1));
+    if (L + 1 < v.layers) {
+      const _Float16 *nw[3] = {lp[16], lp[18], lp[20]}, *nb[3] = {lp[17], lp[19], lp[21]};  // the next layer's q/k/v
+      ahead = beside(a2, args(hn, nw, nb, 3, 3 * H, H, qkv, ME_STORE));
+    } else {
+      ahead = beside(a2, ap);
+    }
     MLCV_TRY(linear(a2));
   }
-  const _Float16* const* tail = prm + 3 + 16 * v.layers;  // post LN w, b; projector w, b
-  const MidArgs ap = args(hn, tail + 2, tail + 3, 1, v.proj, H, out, ME_STORE);
-  MLCV_TRY(layernorm(x, tail[0], tail[1], np, H, v.eps, hn, prefetch({&ap}, LN_PF), st));
+  MLCV_TRY(layernorm(x, tail[0], tail[1], np, H, v.eps, hn, ahead ? Prefetch{} : prefetch({&ap}, LN_PF), st));
   return linear(ap);
 }
 
