@@ -16,7 +16,7 @@
 // 128 x 128 tiles over 3 K slices that met in the kernel, then an epilogue launch of 3 to 5 us per
 // matrix): q/k/v 1152 -> 3456 in 8.8 (16.8 + 3 x 4.7), out_proj 1152 -> 1152 in 6.4 (14.2 + 4.7), fc1
 // 1152 -> 4304 in 11.8 (20.1 + 4.7), fc2 4304 -> 1152 in 14.9 (20.1 + 4.7).  Tried at these sizes: 16 waves
-// that own 32 x 32 blocks of a shared ring (fc1 10.6, out_proj 7.5, the tower 1718 us against 1714 now),
+// that own 32 x 32 blocks of a shared ring (fc1 10.6, out_proj 7.5, the tower 1718 us against 1714),
 // K split over 4 waves of a 128 x 64 tile 2 (fc1 17.1), operands through registers instead of DMA (the
 // tower 2022), each workgroup prefetching its own weights first (1893 against 1826 then).
 #include "kernels.h"
