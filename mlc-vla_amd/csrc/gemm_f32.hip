@@ -20,6 +20,7 @@
 // 2.2 to 5 us in all.  Two layers' prefill 13.08 -> 2.95 ms, the small model's chunk 4.04 -> 0.62 ms (1.87 and
 // 0.46 ms with the attention on the matrix cores and the captured chunk).
 #include "f32.h"
+#include "plan.h"
 
 #include <algorithm>
 
@@ -498,11 +499,7 @@ int f32_gemm_launch(const F32Op& in, hipStream_t st) {
   MLCV_REQUIRE(a.x && a.M > 0 && a.K > 0 && a.N > 0 && a.K % 8 == 0 && a.N % 8 == 0 && a.ldx % 4 == 0,
                "float32 linear: shape");
   const int cus = std::max(device_cus(), 1);
-  const long t128 = (long)((a.M + 127) / 128) * ((a.N + 127) / 128);
-  const long t64 = (long)((a.M + 63) / 64) * ((a.N + 63) / 64);
-  // tiles where they fill the CUs (128 x 128 twice over: half the LDS traffic per flop); below that
-  // 16-row slabs whose waves share out K
-  const int bm = a.M > 64 && t128 >= 2 * cus ? 128 : a.M > 32 && t64 >= cus ? 64 : 0;
+  const int bm = f32_tile(a.M, a.N, a.tab != nullptr, cus);
   int norm = a.nw ? 1 : a.mod ? 2 : 0;
   const bool fuse = bm == 0 && !a.tab;  // in the skinny kernel's one pass; a launch before the tiles
   if (norm != 0 && !fuse) {
@@ -514,7 +511,6 @@ int f32_gemm_launch(const F32Op& in, hipStream_t st) {
     norm = 0;
   }
   if (bm) {
-    MLCV_REQUIRE(!a.tab, "float32 linear: tables run on the skinny kernel");
     switch (a.epi) {
       case FE_STORE: return tile_launch<FE_STORE>(a, bm, st);
       case FE_QKV: return tile_launch<FE_QKV>(a, bm, st);

@@ -52,6 +52,17 @@ inline size_t f32_attn_ws_floats(int KV, int rows, int hd, int nsplit) {
   return nsplit > 1 ? (size_t)KV * nsplit * rpad * (hd + 2) : 0;
 }
 
+// ---- float32 linears (gemm_f32.hip) ---------------------------------------------------------
+// Tile edge of the many-row kernel, or 0 for the few-row kernel's 16-row slabs: tiles where they fill the
+// CUs (128 x 128 twice over: half the LDS traffic per flop).  Equally shaped linears over the same rows (a
+// table: the modulations of up to 64 steps) are slabs at any size, the kernel that takes them all in one
+// launch.
+inline int f32_tile(int M, int N, bool table, int cus) {
+  const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128), t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
+  if (table) return 0;
+  return M > 64 && t128 >= 2L * cus ? 128 : M > 32 && t64 >= cus ? 64 : 0;
+}
+
 // ---- skinny GEMM (gemm_skinny.hip) ------------------------------------------------------
 constexpr int SK_KC = 128;        // k per chunk
 constexpr int SK_MAX_SPLIT = 8;   // K slices at most

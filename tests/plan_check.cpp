@@ -78,6 +78,21 @@ static void check_f32_attn() {
       }
 }
 
+// A float32 table launch (the modulations of up to 64 steps) takes the few-row kernel at any width and
+// device size; a plain one takes tiles where they fill the CUs
+static void check_f32_tile() {
+  for (int cus : {8, 32, 64, 256, 304})
+    for (int M : {1, 16, 32, 33, 64, 65, 968})
+      for (int N : {8, 192, 3072, 16368, 65536}) {
+        ++checked;
+        CHECK(f32_tile(M, N, true, cus) == 0, "table M %d N %d cus %d on tiles", M, N, cus);
+        const int bm = f32_tile(M, N, false, cus);
+        CHECK(bm == 0 || (M > bm / 2 && (long)((M + bm - 1) / bm) * ((N + bm - 1) / bm) >= (bm == 128 ? 2L : 1L) * cus),
+              "M %d N %d cus %d: tile %d", M, N, cus, bm);
+      }
+  CHECK(f32_tile(100, 8192, false, 256) == 64 && f32_tile(150, 32768, false, 256) == 128, "gate_up tiles");
+}
+
 static void check_skinny() {
   for (int ntiles : {1, 2, 3, 8, 16, 40, 64, 160, 256, 512, 1024})
     for (int K : {32, 96, 128, 129, 512, 1024, 2048, 4096, 16384})
@@ -199,6 +214,7 @@ static void check_tile() {
 int main() {
   check_attn();
   check_f32_attn();
+  check_f32_tile();
   check_skinny();
   check_modulations();
   check_mid();

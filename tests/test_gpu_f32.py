@@ -5,6 +5,7 @@ from __future__ import annotations
 
 import numpy as np
 import pytest
+import torch
 
 from conftest import cosine
 from mlc_vla import runtime
@@ -82,3 +83,64 @@ def test_f32_model_vs_oracle(shape):
              for _ in range(2)]
     _tol(chunk[0], loop.numpy(), "chunk")
     np.testing.assert_array_equal(chunk[1], chunk[0])
+
+
+def _model(width, depth, heads, kv, hd, P, T, steps):
+    """A float32 configuration with action width `width` and `steps` Euler steps."""
+    expert = dict(depth=depth, num_heads=heads, num_kv_heads=kv, head_dim=hd)
+    return Pi0Config(paligemma_variant=GemmaExpertConfig(width=64, mlp_dim=64, **expert),
+                     action_expert_variant=GemmaExpertConfig(width=width, mlp_dim=64, **expert), image_keys=(),
+                     max_token_len=P, action_horizon=T, action_dim=32, num_denoise_steps=steps, dtype="float32")
+
+
+@pytest.mark.parametrize("steps", [1, 17, 33, 65])
+def test_f32_loop_step_counts(steps):
+    """Modulations of several steps as one product: one to four row tiles per workgroup (width 1368), and the
+    steps past the 64 that are made at once."""
+    print(f"float32 loop of {steps} steps", flush=True)
+    cfg = _model(1368, 1, 2, 1, 16, 40, 3, steps)
+    d = O.dims_from_config(cfg)
+    runner = PiZeroRunner(cfg, "rocm")
+    p = O.make_params(O.param_specs(d), steps, "float32")
+    params = [runtime.tensor(p[n], runner.dev) for n, _ in runner.named_params]
+    rng = np.random.default_rng(steps)
+    keys, values = (rng.standard_normal((1, 1, 1, 40, 16)).astype(np.float32) for _ in range(2))
+    x = rng.standard_normal((1, 3, 32)).astype(np.float32)
+    cos, sin = make_rope_np(3, 16, 10_000.0, offset=33)
+    te = np.concatenate(make_time_embs(steps, 1368), 0).astype(np.float32)
+    args = (keys, values, x, te, cos, sin, make_prefix_mask_np(40, num_valid=33))
+    ref = O.denoise_loop_kv(p, d, *args, O.Prec("f32"))
+    for graph in (False, True):
+        runner.vm.set_graph(graph)
+        got = runner.vm["denoise_loop_kv"](*(runtime.tensor(a, runner.dev) for a in args), params)
+        _tol(got.numpy(), ref, f"{steps} steps, graph {graph}")
+
+
+def test_f32_loop_wide_modulations():
+    """33 steps at action width 5456, whose 256 column tiles of 64 would fill the CUs: the loop against its own
+    steps, whose modulations are one row."""
+    print("float32 loop, width 5456", flush=True)
+    steps, width = 33, 5456
+    cfg = _model(width, 1, 1, 1, 16, 40, 2, steps)
+    runner = PiZeroRunner(cfg, "rocm")
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    shared = {}  # equal shapes share their weights
+
+    def weight(shape):
+        if shape not in shared:
+            shared[shape] = runtime.Tensor(0.02 * torch.randn(shape, device="cuda", generator=gen), "float32")
+        return shared[shape]
+
+    params = [weight(tuple(sp.shape)) for _, sp in runner.named_params]
+    dv = lambda a: runtime.tensor(np.ascontiguousarray(a, np.float32), runner.dev)  # noqa: E731
+    rng = np.random.default_rng(3)
+    keys, values = (dv(rng.standard_normal((1, 1, 1, 40, 16))) for _ in range(2))
+    x = rng.standard_normal((1, 2, 32)).astype(np.float32)
+    cos, sin = (dv(a) for a in make_rope_np(2, 16, 10_000.0, offset=33))
+    te = np.concatenate(make_time_embs(steps, width), 0).astype(np.float32)
+    pm = dv(make_prefix_mask_np(40, num_valid=33))
+    got = runner.vm["denoise_loop_kv"](keys, values, dv(x), dv(te), cos, sin, pm, params).numpy()
+    for i in range(steps):
+        v = runner.vm["denoise_step_kv"](keys, values, dv(x), dv(te[i:i + 1]), cos, sin, pm, params).numpy()
+        x = x + np.float32(-1.0 / steps) * v
+    _tol(got, x, "loop")
