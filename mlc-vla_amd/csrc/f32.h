@@ -29,7 +29,7 @@ struct F32Op {
   int ldx, M, K, N;
   const float* w[3];       // FE_QKV: q, k, v; else w[0]
   const float* b;          // [N] or null
-  const F32Tab* tab;       // ntab linears over the same x: w, b from the table, out + z * tab_stride
+  const F32Tab* tab;       // (host) ntab linears over the same x: w, b from the table, out + z * tab_stride
   int ntab;
   size_t tab_stride;
   // x is normalised first: x / sqrt(mean(x^2) + eps), then * (1 + nw) (RMSNorm) or

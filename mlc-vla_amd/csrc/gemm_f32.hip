@@ -297,21 +297,15 @@ constexpr int FS_NW = 8;  // waves: each takes every 8th block of 32 k
 // the rows' sums of squares are added up on the way, and y = product / sqrt(mean(x^2) + eps) + shift . w.
 // A launch is a chain of memory latencies, so everything it reads goes out before the first wait: the
 // first blocks of the weights and of x, then what the epilogue reads.
+// w0, b, out: the operation's own, or those of one linear of a table.
 template <int MT, int NORM, int EPI>
-__global__ __launch_bounds__(64 * FS_NW) void f32_skinny_kernel(const F32Op a) {
+__device__ __forceinline__ void f32_skinny(const F32Op& a, const float* w0, const float* b, float* out) {
   __shared__ f4 red[FS_NW * MT * 64];
   __shared__ float ssq[NORM != 0 ? FS_NW * MT * 16 : 1];  // sums of squares [wave][row]
   __shared__ float shw[NORM == 2 ? FS_NW * 16 : 1];       // shift . w [wave][weight row]
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
   const int m0 = blockIdx.y * 16 * MT, K = a.K;
-  const float *w0 = a.w[0], *b = a.b;
-  float* out = a.out;
-  if (a.tab) {
-    w0 = a.tab[blockIdx.z].w;
-    b = a.tab[blockIdx.z].b;
-    out += blockIdx.z * a.tab_stride;
-  }
   const float* wr = w_row<EPI>(a, w0, min(16 * (int)blockIdx.x + r, a.N - 1));
   const float* xr[MT];
 #pragma unroll
@@ -437,6 +431,23 @@ __global__ __launch_bounds__(64 * FS_NW) void f32_skinny_kernel(const F32Op a) {
   }
 }
 
+template <int MT, int NORM, int EPI>
+__global__ __launch_bounds__(64 * FS_NW) void f32_skinny_kernel(const F32Op a) {
+  f32_skinny<MT, NORM, EPI>(a, a.w[0], a.b, a.out);
+}
+
+// The linears of a table, grid z.  The pointers are kernel arguments, as every other launch's: a launch
+// that a caller has captured keeps the weights it was captured with.
+constexpr int FS_TAB = 64;  // linears per launch
+struct F32Tabs {
+  F32Tab t[FS_TAB];
+};
+template <int MT>
+__global__ __launch_bounds__(64 * FS_NW) void f32_skinny_tab_kernel(const F32Op a, const F32Tabs tabs) {
+  const int z = blockIdx.z;
+  f32_skinny<MT, 0, FE_STORE>(a, tabs.t[z].w, tabs.t[z].b, a.out + z * a.tab_stride);
+}
+
 // one row per workgroup: xn = x / sqrt(mean(x^2) + eps), then * (1 + w) or * (1 + mod) + mod[K + ..]
 __global__ __launch_bounds__(256) void f32_rows_norm_kernel(const float* __restrict__ x, int ldx, int K,
                                                             const float* __restrict__ nw,
@@ -484,11 +495,28 @@ int tile_launch(const F32Op& a, int bm, hipStream_t st) {
 
 template <int NORM, int EPI>
 int skinny_launch(const F32Op& a, int mt, hipStream_t st) {
-  const dim3 grid((a.N + 15) / 16, (a.M + 16 * mt - 1) / (16 * mt), a.tab ? a.ntab : 1);
+  const dim3 grid((a.N + 15) / 16, (a.M + 16 * mt - 1) / (16 * mt));
   if (mt == 1) f32_skinny_kernel<1, NORM, EPI><<<grid, 64 * FS_NW, 0, st>>>(a);
   else if (mt == 2) f32_skinny_kernel<2, NORM, EPI><<<grid, 64 * FS_NW, 0, st>>>(a);
   else f32_skinny_kernel<4, NORM, EPI><<<grid, 64 * FS_NW, 0, st>>>(a);
   MLCV_HIP(hipGetLastError());
+  return 0;
+}
+
+int tab_launch(const F32Op& in, int mt, hipStream_t st) {
+  for (int i = 0; i < in.ntab; i += FS_TAB) {
+    F32Op a = in;
+    F32Tabs tabs{};
+    const int n = std::min(FS_TAB, in.ntab - i);
+    std::copy(in.tab + i, in.tab + i + n, tabs.t);
+    a.out = in.out + i * in.tab_stride;
+    a.tab = nullptr;  // the host's
+    const dim3 grid((a.N + 15) / 16, (a.M + 16 * mt - 1) / (16 * mt), n);
+    if (mt == 1) f32_skinny_tab_kernel<1><<<grid, 64 * FS_NW, 0, st>>>(a, tabs);
+    else if (mt == 2) f32_skinny_tab_kernel<2><<<grid, 64 * FS_NW, 0, st>>>(a, tabs);
+    else f32_skinny_tab_kernel<4><<<grid, 64 * FS_NW, 0, st>>>(a, tabs);
+    MLCV_HIP(hipGetLastError());
+  }
   return 0;
 }
 
@@ -498,10 +526,11 @@ int f32_gemm_launch(const F32Op& in, hipStream_t st) {
   F32Op a = in;
   MLCV_REQUIRE(a.x && a.M > 0 && a.K > 0 && a.N > 0 && a.K % 8 == 0 && a.N % 8 == 0 && a.ldx % 4 == 0,
                "float32 linear: shape");
+  MLCV_REQUIRE(!a.tab || (a.ntab > 0 && a.epi == FE_STORE && !a.nw && !a.mod), "float32 linear: table");
   const int cus = std::max(device_cus(), 1);
   const int bm = f32_tile(a.M, a.N, a.tab != nullptr, cus);
   int norm = a.nw ? 1 : a.mod ? 2 : 0;
-  const bool fuse = bm == 0 && !a.tab;  // in the skinny kernel's one pass; a launch before the tiles
+  const bool fuse = bm == 0;  // in the skinny kernel's one pass; a launch before the tiles
   if (norm != 0 && !fuse) {
     MLCV_REQUIRE(a.xn, "float32 linear: no room for the normalised rows");
     f32_rows_norm_kernel<<<a.M, 256, 0, st>>>(a.x, a.ldx, a.K, a.nw, a.mod, a.eps, a.xn);
@@ -523,6 +552,7 @@ int f32_gemm_launch(const F32Op& in, hipStream_t st) {
   // m tiles of 16 rows per workgroup: up to 4, fewer while the grid would leave CUs idle
   int mt = a.M <= 16 ? 1 : a.M <= 32 ? 2 : 4;
   while (mt > 1 && (long)((a.N + 15) / 16) * ((a.M + 16 * mt - 1) / (16 * mt)) < cus) mt >>= 1;
+  if (a.tab) return tab_launch(a, mt, st);
   switch (a.epi) {
     case FE_STORE: return norm == 2 ? skinny_launch<2, FE_STORE>(a, mt, st) : norm == 1 ? skinny_launch<1, FE_STORE>(a, mt, st) : skinny_launch<0, FE_STORE>(a, mt, st);
     case FE_QKV: return norm == 2 ? skinny_launch<2, FE_QKV>(a, mt, st) : norm == 1 ? skinny_launch<1, FE_QKV>(a, mt, st) : skinny_launch<0, FE_QKV>(a, mt, st);

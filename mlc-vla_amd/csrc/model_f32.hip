@@ -244,7 +244,7 @@ struct F32Model {
   bool bound = false;
   // the matrix-core kernels (gemm_f32.hip) take these widths and weight pointers; else the general ones
   bool shape_ok = false, fast = false;
-  F32Tab* tab = nullptr;  // the 2 D + 1 modulations' weights and biases (device)
+  std::vector<F32Tab> tab;  // the 2 D + 1 modulations' weights and biases
   // the loop and the chunk as captured graphs over the model's own buffers (MLCV_OPT_USE_GRAPH): the
   // inputs are staged into them and the caller's cache is reached through kvp, so a graph serves
   // every call until the parameters are bound again
@@ -267,7 +267,6 @@ struct F32Model {
 
   ~F32Model() {
     for (void* p : owned) (void)hipFree(p);
-    if (tab) (void)hipFree(tab);
     if (kvp) (void)hipFree(kvp);
     drop_graphs();
     if (cap) (void)hipStreamDestroy(cap);
@@ -400,7 +399,7 @@ int f32_mods(F32Model& m, const float* te, int steps, hipStream_t st) {
   a.act = 1;
   MLCV_TRY(f32_gemm_launch(a, st));
   a = lin_op(m.cond, W1, steps, m.final_mod, FE_STORE, m.mods, nm * 3 * W1);
-  a.tab = m.tab;
+  a.tab = m.tab.data();
   a.ntab = nm;
   a.tab_stride = (size_t)3 * W1;
   return f32_gemm_launch(a, st);
@@ -661,12 +660,10 @@ int f32_bind(F32Model& m, const void* const* ptrs, int count) {
   m.fast = m.shape_ok;
   for (int i = 0; i < count; ++i) m.fast = m.fast && f32_aligned({ptrs[i]});
   if (m.fast) {
-    std::vector<F32Tab> tab;
+    m.tab.clear();
     for (const F32Layer& ly : m.layers)
-      for (const F32Lin* l : {&ly.mod_in, &ly.mod_post}) tab.push_back({l->w, l->b});
-    tab.push_back({m.final_mod.w, m.final_mod.b});
-    if (!m.tab) MLCV_HIP(hipMalloc(reinterpret_cast<void**>(&m.tab), tab.size() * sizeof(F32Tab)));
-    MLCV_HIP(hipMemcpy(m.tab, tab.data(), tab.size() * sizeof(F32Tab), hipMemcpyHostToDevice));
+      for (const F32Lin* l : {&ly.mod_in, &ly.mod_post}) m.tab.push_back({l->w, l->b});
+    m.tab.push_back({m.final_mod.w, m.final_mod.b});
   }
   m.bound = true;
   return 0;

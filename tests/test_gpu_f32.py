@@ -144,3 +144,54 @@ def test_f32_loop_wide_modulations():
         v = runner.vm["denoise_step_kv"](keys, values, dv(x), dv(te[i:i + 1]), cos, sin, pm, params).numpy()
         x = x + np.float32(-1.0 / steps) * v
     _tol(got, x, "loop")
+
+
+def _loop_case(cfg, seed, dv):
+    """Random arguments of denoise_loop_kv (keys, values, x0, time embeddings, RoPE, mask), on the device by dv."""
+    e, P, T = cfg.action_expert, cfg.prefix_len, cfg.suffix_len
+    rng = np.random.default_rng(seed)
+    valid = int(rng.integers(P // 2, P + 1))
+    kv = (e.depth, 1, e.num_kv_heads, P, e.head_dim)
+    te = np.concatenate(make_time_embs(cfg.num_denoise_steps, e.width), 0) + 0.01 * rng.standard_normal((1, e.width))
+    cos, sin = make_rope_np(T, e.head_dim, 10_000.0, offset=valid)
+    return [dv(a) for a in (rng.standard_normal(kv), rng.standard_normal(kv), rng.standard_normal((1, T, 32)), te, cos,
+                            sin, make_prefix_mask_np(P, num_valid=valid))]
+
+
+def test_f32_many_layers():
+    """More modulations than one launch takes (33 layers: 67 of them), against the oracle."""
+    print("float32 loop of 33 layers", flush=True)
+    cfg = _model(64, 33, 2, 1, 16, 40, 3, 3)
+    d = O.dims_from_config(cfg)
+    runner = PiZeroRunner(cfg, "rocm")
+    p = O.make_params(O.param_specs(d), 1, "float32")
+    dv = lambda a: runtime.tensor(np.ascontiguousarray(a, np.float32), runner.dev)  # noqa: E731
+    args = _loop_case(cfg, 1, dv)
+    ref = O.denoise_loop_kv(p, d, *(a.numpy() for a in args), O.Prec("f32"))
+    got = runner.vm["denoise_loop_kv"](*args, [dv(p[n]) for n, _ in runner.named_params])
+    _tol(got.numpy(), ref, "33 layers")
+
+
+def test_f32_captured_loop_keeps_its_parameters():
+    """A loop that a caller captured goes on with the parameters it was captured with after others are bound."""
+    print("float32 loop captured by the caller", flush=True)
+    cfg = _model(64, 2, 2, 1, 32, 40, 3, 3)
+    d = O.dims_from_config(cfg)
+    runner = PiZeroRunner(cfg, "rocm")
+    loop = runner.vm["denoise_loop_kv"]
+    dv = lambda a: runtime.tensor(np.ascontiguousarray(a, np.float32), runner.dev)  # noqa: E731
+    first, second = ([dv(p[n]) for n, _ in runner.named_params]
+                     for p in (O.make_params(O.param_specs(d), seed, "float32") for seed in (1, 2)))
+    args, other = _loop_case(cfg, 1, dv), _loop_case(cfg, 2, dv)
+    ref = loop(*args, first).numpy()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out = loop(*args, first)
+    for params in (first, second, first):
+        between = loop(*other, params).numpy()  # another eager call, and the bind of its parameters
+        out.torch.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out.numpy(), ref)
+        assert np.abs(between - ref).max() > 1e-3
