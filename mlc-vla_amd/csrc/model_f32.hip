@@ -613,13 +613,12 @@ int f32_create(const ::mlcv_config& cfg, F32Model** out) {
 
 void f32_destroy(F32Model* m) { delete m; }
 
-void f32_set_graph(F32Model& m, bool on) {
-  m.use_graph = on;
-  m.drop_graphs();
-}
+void f32_set_graph(F32Model& m, bool on) { m.use_graph = on; }
 
 int f32_bind(F32Model& m, const void* const* ptrs, int count) {
   m.bound = false;
+  // a replay may still be running on any stream: the call that started it did not wait
+  if (m.g_loop || m.g_chunk) MLCV_HIP(hipDeviceSynchronize());
   m.drop_graphs();
   int idx = 0;
   auto f = [&]() { return reinterpret_cast<const float*>(ptrs[idx++]); };

@@ -195,3 +195,27 @@ def test_f32_captured_loop_keeps_its_parameters():
         torch.cuda.synchronize()
         np.testing.assert_array_equal(out.numpy(), ref)
         assert np.abs(between - ref).max() > 1e-3
+
+
+def test_f32_replay_outlives_options_and_binds():
+    """Options set and other parameters bound while a replayed loop runs on another stream leave it alone."""
+    print("float32 replay in flight", flush=True)
+    cfg = _model(64, 33, 2, 1, 32, 40, 3, 60)
+    d = O.dims_from_config(cfg)
+    runner = PiZeroRunner(cfg, "rocm", cuda_graph=True)
+    vm = runner.vm
+    dv = lambda a: runtime.tensor(np.ascontiguousarray(a, np.float32), runner.dev)  # noqa: E731
+    first, second = ([dv(p[n]) for n, _ in runner.named_params]
+                     for p in (O.make_params(O.param_specs(d), seed, "float32") for seed in (1, 2)))
+    args = _loop_case(cfg, 1, dv)
+    refs = [vm["denoise_loop_kv"](*args, params).numpy() for params in (second, first)]
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    for change in (lambda: vm.set_graph(True), lambda: vm.set_graph(False), lambda: vm._bind(second)):
+        vm.set_graph(True)
+        with torch.cuda.stream(side):
+            out = vm["denoise_loop_kv"](*args, first)
+        change()
+        side.synchronize()
+        np.testing.assert_array_equal(out.numpy(), refs[1])
+    np.testing.assert_array_equal(vm["denoise_loop_kv"](*args, second).numpy(), refs[0])
