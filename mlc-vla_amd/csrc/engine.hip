@@ -2448,6 +2448,7 @@ int mlcv_linear(const void* x, int32_t M, int32_t K, const void* w, const uint32
                 const void* bias, void* y, int32_t N, void* stream) {
   MLCV_REQUIRE(x && y && M > 0 && K > 0 && N > 0, "bad argument");
   MLCV_REQUIRE((w != nullptr) != (q_weight != nullptr && q_scale != nullptr), "pass either w or q_weight+q_scale");
+  if (w) q_weight = nullptr;  // words without their scales beside w
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   MidArgs mid;
   if (linear_mid(x, M, K, w, bias, y, N, &mid)) {
@@ -2501,6 +2502,7 @@ int mlcv_linear_noalloc(const void* x, int32_t M, int32_t K, const void* w, cons
                         const void* q_scale, const void* bias, void* y, int32_t N, void* stream) {
   MLCV_REQUIRE(x && y && M > 0 && K > 0 && N > 0, "bad argument");
   MLCV_REQUIRE((w != nullptr) != (q_weight != nullptr && q_scale != nullptr), "pass either w or q_weight+q_scale");
+  if (w) q_weight = nullptr;  // words without their scales beside w
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const int ntiles = (N + 63) / 64, mb = (M + 63) / 64;
   const SkPlan p = sk_plan(ntiles, K, mb, 0);

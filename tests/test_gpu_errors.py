@@ -8,7 +8,8 @@ again afterwards.
   mlcv_sync when the keys are read.
 
 Also: a failed mlcv_bind_params leaves the context unbound, so a caller that still believes
-the old binding stands gets "parameters not bound" instead of a step over freed copies.
+the old binding stands gets "parameters not bound" instead of a step over freed copies; and a linear given
+stray q4f16_1 words beside its fp16 weights.
 """
 
 from __future__ import annotations
@@ -95,3 +96,19 @@ def test_failed_bind_leaves_the_context_unbound():
         s.run()
     vm._bound = None  # a caller that binds again gets the same results as before
     np.testing.assert_array_equal(s.run(), good)
+
+
+@pytest.mark.parametrize("fn", ["mlcv_linear", "mlcv_linear_noalloc"])
+@pytest.mark.parametrize("m,k,n", [(16, 512, 64), (16, 4096, 64), (80, 512, 64), (80, 128, 64)])
+def test_linear_words_without_scales_beside_fp16_weights(fn, m, k, n):
+    """q_weight without q_scale beside w is an fp16 linear on every route: no kernel takes it for q4f16_1 and
+    reads the scales that are not there."""
+    print(f"{fn} M={m} K={k} N={n} with stray words", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(m + k)
+    x, w = (torch.randn(s, device="cuda", generator=gen).half() for s in ((m, k), (n, k)))
+    words = torch.zeros((n, k // 8), dtype=torch.int32, device="cuda")
+    y, ref = (torch.empty((m, n), dtype=torch.float16, device="cuda") for _ in range(2))
+    N.call(fn, _p(x), m, k, _p(w), None, None, None, _p(ref), n, _st())
+    N.call(fn, _p(x), m, k, _p(w), _p(words), None, None, _p(y), n, _st())
+    torch.cuda.synchronize()
+    assert torch.equal(y, ref)
