@@ -2400,12 +2400,7 @@ int mlcv_tile_linear(const void* x, int32_t M, int32_t K, const void* w, int32_t
   return tile_meet_failed(gerr, "mlcv_tile_linear");
 }
 
-// fp16 linears the mid-size kernel runs instead of the skinny one, which reads the weights once per 64
-// rows: from 65 rows on, K above 256.  Kernel times, skinny / mid, over 248 shapes of 65 to 1100 rows:
-// faster in all with K > 256 (100 x 2048 x 2048: 9.7 / 6.1 us, 457 x 2048 x 2560: 30.4 / 14.3,
-// 968 x 2048 x 2560: 46.5 / 26.2, 200 x 16384 x 2048: 95 / 37, 80 x 16384 x 1024: 29.0 / 26.6, the
-// closest), but 5.0 / 5.4 at 200 x 256 x 4096 and 4.9 / 8.7 at 968 x 64 x 2048, where the mid kernel's
-// start and its meeting outweigh its loop.
+// fp16 linears that the mid-size kernel runs instead of the skinny one (mid_linear)
 static bool linear_mid(const void* x, int32_t M, int32_t K, const void* w, const void* bias, void* y, int32_t N,
                        MidArgs* a) {
   *a = MidArgs{};
@@ -2421,7 +2416,7 @@ static bool linear_mid(const void* x, int32_t M, int32_t K, const void* w, const
   a->y = reinterpret_cast<_Float16*>(y);
   a->ldy = N;
   a->epi = ME_STORE;
-  return w != nullptr && M > 64 && K > 256 && K % 32 == 0 && mid_ok(*a);
+  return w != nullptr && mid_linear(M, K, N, std::max(device_cus(), 1)) && mid_ok(*a);
 }
 
 // Linears that lin_rows_kernel runs instead of the skinny kernel: one round of workgroups, and rows x K up

@@ -138,6 +138,39 @@ static void check_mid() {
       }
 }
 
+// fp16 linears on the mid-size kernel: never below its row count and depth, or where the kernel times
+// (us, skinny / mid) say that it is the slower one
+static void check_mid_linear() {
+  struct Shape {
+    int M, K, N;
+    bool in;
+  };
+  const Shape shapes[] = {
+      {457, 2048, 2560, true},   // 30.4 / 14.3
+      {256, 512, 4096, true},    // 7.6 / 6.4: one round
+      {968, 512, 4096, false},   // 17.6 / 20.4: two
+      {457, 288, 16384, false},  // 26.0 / 35.8
+      {83, 416, 15748, false},   // 9.5 / 11.2
+      {968, 768, 16384, true},   // 106.8 / 78.1
+      {942, 672, 2128, false},   // 14.4 / 15.9: rows across lines
+      {582, 928, 2908, true},    // 17.6 / 14.1
+      {640, 8192, 64, true},     // 16.3 / 14.0
+      {1100, 8192, 64, false},   // 19.8 / 24.3: an XCD or two
+      {1226, 14112, 256, false}, // 49.1 / 57.1
+      {285, 7968, 64, false},    // 14.5 / 16.4: rows across lines
+      {126, 16160, 28, false},   // 21.4 / 25.3
+      {801, 3328, 32, true},     // 11.2 / 8.1
+      {3846, 800, 2324, false},  // 55.8 / 65.0
+      {16384, 512, 256, false},  // 19.5 / 42.2
+      {64, 2048, 2048, false},   // the skinny kernel's rows
+      {200, 256, 4096, false},
+  };
+  for (const Shape& s : shapes) {
+    ++checked;
+    CHECK(mid_linear(s.M, s.K, s.N, 256) == s.in, "linear %d x %d x %d", s.M, s.K, s.N);
+  }
+}
+
 // The modulation pieces of mlcv_bind_params on 64-row tiles (layer 0's two norms, then the other
 // NM - 2, 3 W1 rows each): the workspace mlcv_create allocates holds the partials of each piece.
 static void check_modulations() {
@@ -218,6 +251,7 @@ int main() {
   check_skinny();
   check_modulations();
   check_mid();
+  check_mid_linear();
   check_tile();
   std::printf("plans checked: %ld, failures: %d\n", checked, failures);
   return failures ? 1 : 0;
