@@ -367,6 +367,8 @@ int mid_spare(const MidArgs& a) {
   return (int)std::max(0L, cus - (nt + TG_NXCD - 1) / TG_NXCD * TG_NXCD * mt);
 }
 
+bool mid_worth(const MidArgs& a) { return mid_vs_tile(a.M, a.N, a.K, std::max(device_cus(), 1)); }
+
 void mid_prefetch_add(const MidArgs& a, int nblocks, Prefetch& pf) {
   if (!mid_ok(a)) return;
   const int plan = mid_plan(a.M, a.N, std::max(device_cus(), 1));

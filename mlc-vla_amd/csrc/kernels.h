@@ -259,6 +259,7 @@ struct MidArgs {
 };
 int mid_spare(const MidArgs& a);  // CUs that its tiles leave idle
 bool mid_ok(const MidArgs& a);  // shapes and alignments the kernel takes
+bool mid_worth(const MidArgs& a);  // faster than the long-M tile GEMM and an epilogue pass
 int mid_gemm_launch(const MidArgs& a, hipStream_t st);
 // the weights of a later mid_gemm_launch of `a`, for `nblocks` prefetch workgroups of an earlier launch
 void mid_prefetch_add(const MidArgs& a, int nblocks, Prefetch& pf);

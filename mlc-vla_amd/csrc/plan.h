@@ -134,6 +134,19 @@ inline int mid_plan(int M, int N, int cus, long* rows = nullptr, long* rounds = 
   return best;
 }
 
+// Linears of the image tower that run on this kernel, not on the long-M tile GEMM (256 rows of 128 or 256
+// outputs, K split) and an epilogue pass.  This kernel's tiles read more operand rows per product and K is not
+// split, so it is the slower one past 1024 rows, in many rounds and at long K.  Towers, us, the tile GEMM and
+// pass / this kernel for all linears: 4 layers of width 1152 of 256 patches 444 / 268, 1024 patches 654 / 646,
+// 1369 patches 894 / 1060.  3 layers, and with this rule: width 1152 of 1024 patches 602 / 457 / 461, 2048 (MLP
+// 8192) of 784 832 / 793 / 746, 3072 (8192) of 784 1064 / 1141 / 1014, 4096 (16384) of 256 889 / 947 / 802 and of
+// 1024 2008 / 2707 / 1975.
+inline bool mid_vs_tile(int M, int N, int K, int cus) {
+  long rows = 0, rounds = 0;
+  mid_plan(M, N, cus, &rows, &rounds);
+  return M <= 1024 && rounds <= 3 && rows * K <= 1400000;
+}
+
 // fp16 linears (mlcv_linear) that run on this kernel, not on the skinny one: the shapes of more than 64
 // rows and K > 256 where it is the faster of the two.  Kernel times over 2800 shapes of 65 to 16384 rows on
 // 256 CUs, skinny / this, us; inside it is 1.01 to 5 times as fast.

@@ -48,11 +48,6 @@ __global__ void pad_cols_kernel(const _Float16* __restrict__ w, int k, int kp, _
 constexpr int LN_PF = 256, ATTN_PF = 128;
 constexpr int MID_PF_MIN = 32;
 
-// Rows up to which a linear runs on gemm_mid.hip's small tiles, else on the long-M GEMM with an epilogue
-// pass.  4 layers of width 1152, us, without / with the small tiles: 256 patches 444 / 268, 1024 patches
-// 654 / 646, 1369 patches 894 / 1060.
-constexpr int MID_MAX_ROWS = 1024;
-
 enum VisEpi { VE_BIAS = 0, VE_BIAS_GELU = 1, VE_BIAS_RESIDUAL = 2, VE_BIAS_POS = 3 };
 
 // y = fp16(y + b) on columns [0, n) of rows with stride ldy, then:
@@ -355,8 +350,11 @@ __global__ __launch_bounds__(256) void vis_attn_kernel(const _Float16* __restric
 int vis_attn(const _Float16* qkv, int T, int H, int hd, _Float16* out, Prefetch pf, hipStream_t st) {
   // Two row tiles a workgroup halve the reads of K and V, where that still leaves a workgroup per CU.  4
   // layers of 16 heads of 72, us, one / two: 256 patches 265 / 276, 576 patches 419 / 415, 1024 patches
-  // 644 / 589, 4096 patches 3738 / 2699.
-  const bool wide = (long)(T + 31) / 32 * H >= std::max(device_cus(), 1) && hd <= 128;
+  // 644 / 589, 4096 patches 3738 / 2699.  Past a head dim of 128 a CU holds one workgroup (256 registers and
+  // more), so two tiles pay as soon as single ones take a second round: 3 layers of 16 heads of 160 1530 / 1329
+  // at 1369 patches, of 4 heads of 256 2186 / 1519 at 4096.
+  const long cus = std::max(device_cus(), 1), one = (long)(T + 15) / 16 * H, two = (long)(T + 31) / 32 * H;
+  const bool wide = hd <= 128 ? two >= cus : one > cus;
   dim3 grid(wide ? (T + 31) / 32 : (T + 15) / 16, H);
   if (pf.nreg > 0) {  // whole grid rows of prefetch workgroups
     const int rows = (pf.nblocks + (int)grid.x - 1) / (int)grid.x;
@@ -381,8 +379,14 @@ int vis_attn(const _Float16* qkv, int T, int H, int hd, _Float16* out, Prefetch 
       if (wide) vis_attn_kernel<4, 2><<<grid, 256, 0, st>>>(qkv, T, H, hd, scale, out, pf);
       else vis_attn_kernel<4, 1><<<grid, 256, 0, st>>>(qkv, T, H, hd, scale, out, pf);
       break;
-    case 5: case 6: vis_attn_kernel<6, 1><<<grid, 256, 0, st>>>(qkv, T, H, hd, scale, out, pf); break;
-    case 7: case 8: vis_attn_kernel<8, 1><<<grid, 256, 0, st>>>(qkv, T, H, hd, scale, out, pf); break;
+    case 5: case 6:
+      if (wide) vis_attn_kernel<6, 2><<<grid, 256, 0, st>>>(qkv, T, H, hd, scale, out, pf);
+      else vis_attn_kernel<6, 1><<<grid, 256, 0, st>>>(qkv, T, H, hd, scale, out, pf);
+      break;
+    case 7: case 8:
+      if (wide) vis_attn_kernel<8, 2><<<grid, 256, 0, st>>>(qkv, T, H, hd, scale, out, pf);
+      else vis_attn_kernel<8, 1><<<grid, 256, 0, st>>>(qkv, T, H, hd, scale, out, pf);
+      break;
     default: MLCV_REQUIRE(false, "vision head_dim above 256");
   }
   MLCV_HIP(hipGetLastError());
@@ -467,8 +471,8 @@ int embed_image_enqueue(const VisionCfg& v, const _Float16* const* prm, const _F
     return 0;
   };
 
-  // y = epilogue(a . [w0 | w1 | w2]^T + bias): fused up to MID_MAX_ROWS rows (and aligned operands), else the
-  // long-M GEMM and a pass
+  // y = epilogue(a . [w0 | w1 | w2]^T + bias): fused on gemm_mid.hip's small tiles where they are the faster
+  // ones (and the operands aligned), else the long-M GEMM and a pass
   auto args = [&](const _Float16* a, const _Float16* const* w, const _Float16* const* b, int nseg, int N, int K,
                   _Float16* y, int epi_mode) {
     MidArgs g{};
@@ -490,8 +494,9 @@ int embed_image_enqueue(const VisionCfg& v, const _Float16* const* prm, const _F
     g.npos = np;
     return g;
   };
+  auto small = [&](const MidArgs& g) { return mid_ok(g) && mid_worth(g); };
   auto linear = [&](const MidArgs& g) -> int {
-    if (np <= MID_MAX_ROWS && mid_ok(g)) return mid_gemm_launch(g, st);
+    if (small(g)) return mid_gemm_launch(g, st);
     _Float16* dst = g.epi == ME_RESIDUAL ? t : g.y;
     MLCV_TRY(gemm(g.x, g.K, g.w[0], g.w[1], g.w[2], g.n1, g.n2, g.K, dst, g.N, np, g.N, g.K));
     const int ve = g.epi == ME_GELU ? VE_BIAS_GELU : g.epi == ME_RESIDUAL ? VE_BIAS_RESIDUAL
@@ -505,14 +510,14 @@ int embed_image_enqueue(const VisionCfg& v, const _Float16* const* prm, const _F
   // launches before it, which are chains of latencies themselves, have them fetched,
   auto prefetch = [&](std::initializer_list<const MidArgs*> ls, int nblocks) {
     Prefetch pf{};
-    if (np <= MID_MAX_ROWS)
-      for (const MidArgs* g : ls) mid_prefetch_add(*g, nblocks, pf);
+    for (const MidArgs* g : ls)
+      if (small(*g)) mid_prefetch_add(*g, nblocks, pf);
     return pf;
   };
   // or, better, those beside an earlier linear, on the CUs that its own tiles leave idle (64 of 256 at fc1 and
   // fc2 of 256 patches): `next`'s weights beside `g`.
   auto beside = [&](MidArgs& g, const MidArgs& next) {
-    const int spare = np <= MID_MAX_ROWS && mid_ok(g) ? mid_spare(g) : 0;
+    const int spare = small(g) ? mid_spare(g) : 0;
     if (spare < MID_PF_MIN) return false;
     g.pf = prefetch({&next}, spare);
     return g.pf.nreg > 0;

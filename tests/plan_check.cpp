@@ -171,6 +171,18 @@ static void check_mid_linear() {
   }
 }
 
+// The image tower's linears on the mid-size kernel, or (many rows, many rounds, long K) on the tile GEMM
+static void check_mid_vs_tile() {
+  for (int M : {4, 64, 196, 256, 576, 1024})
+    for (int N : {1152, 3456, 4304, 2048}) {
+      ++checked;
+      CHECK(mid_vs_tile(M, N, N == 1152 ? 4304 : 1152, 256), "So400m linear %d x %d", M, N);
+    }
+  CHECK(!mid_vs_tile(1025, 1152, 1152, 256), "rows");
+  CHECK(mid_vs_tile(784, 6144, 1152, 256) == false && mid_vs_tile(289, 16384, 64, 256) == false, "rounds");
+  CHECK(!mid_vs_tile(256, 4096, 16384, 256) && !mid_vs_tile(784, 4096, 4096, 256), "long K");
+}
+
 // The modulation pieces of mlcv_bind_params on 64-row tiles (layer 0's two norms, then the other
 // NM - 2, 3 W1 rows each): the workspace mlcv_create allocates holds the partials of each piece.
 static void check_modulations() {
@@ -252,6 +264,7 @@ int main() {
   check_modulations();
   check_mid();
   check_mid_linear();
+  check_mid_vs_tile();
   check_tile();
   std::printf("plans checked: %ld, failures: %d\n", checked, failures);
   return failures ? 1 : 0;

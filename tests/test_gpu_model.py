@@ -231,7 +231,11 @@ def test_vm_embed_image_vs_oracle(sig, tiny):
     (dict(image_size=48, patch_size=2, hidden_size=544, intermediate_size=64, num_attention_heads=16, projection_dim=64), 0),
     (dict(image_size=42, hidden_size=1600, intermediate_size=64, num_attention_heads=20, projection_dim=64), 0),
     (dict(image_size=42, hidden_size=144, intermediate_size=200, num_attention_heads=2, projection_dim=64), 1),
-], ids=["hd5_4p", "hd12_25p", "hd144_16p", "hd256_9p", "hd40_289p", "hd8_1024p", "hd32_1089p", "hd34_576p", "ln1600", "off2bytes"])
+    (dict(image_size=34, patch_size=2, hidden_size=64, intermediate_size=16384, num_attention_heads=2, projection_dim=64), 0),
+    (dict(image_size=66, patch_size=2, hidden_size=576, intermediate_size=64, num_attention_heads=4, projection_dim=64), 0),
+    (dict(image_size=66, patch_size=2, hidden_size=1024, intermediate_size=64, num_attention_heads=4, projection_dim=64), 0),
+], ids=["hd5_4p", "hd12_25p", "hd144_16p", "hd256_9p", "hd40_289p", "hd8_1024p", "hd32_1089p", "hd34_576p", "ln1600", "off2bytes", "mlp16384_289p",
+        "hd144_1089p", "hd256_1089p"])
 def test_vm_embed_image_shapes(sig, off, tiny):
     """embed_image where its kernels have edges: head dims without 8-wide loads and up to 256, partial row
     tiles and key chunks, widths with K and N tails, both LayerNorm register sizes, more than 1024 patches
