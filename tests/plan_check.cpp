@@ -90,7 +90,10 @@ static void check_f32_tile() {
         CHECK(bm == 0 || (M > bm / 2 && (long)((M + bm - 1) / bm) * ((N + bm - 1) / bm) >= (bm == 128 ? 2L : 1L) * cus),
               "M %d N %d cus %d: tile %d", M, N, cus, bm);
       }
+  // what test_gpu_f32.py's shapes are there for, on 256 CUs
   CHECK(f32_tile(100, 8192, false, 256) == 64 && f32_tile(150, 32768, false, 256) == 128, "gate_up tiles");
+  CHECK(f32_tile(520, 2112, false, 256) == 64 && f32_tile(520, 2056, false, 256) == 64, "q/k/v, o_proj and down tiles");
+  CHECK(f32_tile(1000, 8448, false, 256) == 128 && f32_tile(1000, 8200, false, 256) == 128, "the same of 128");
 }
 
 static void check_skinny() {

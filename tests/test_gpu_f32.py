@@ -36,6 +36,9 @@ SHAPES = [
     (64, 16384, 64, 64, 1, 1, 256, 150, 150, 5, 0),   # 128 x 128 tiles (256 x 2), a partial m tile
     (100, 60, 36, 52, 3, 1, 20, 40, 33, 6, 0),        # widths and head dim only the general kernels take
     (64, 128, 64, 128, 2, 1, 32, 40, 33, 6, 1),       # misaligned weights and inputs
+    (2056, 64, 64, 64, 11, 11, 64, 520, 500, 3, 0),   # q/k/v, o_proj and down on 64 x 64 tiles, N of 8 mod 16
+    (8200, 64, 64, 64, 1, 1, 16, 1000, 900, 2, 0),    # o_proj and down on 128 x 128 tiles, a partial one each way
+    (72, 64, 64, 64, 11, 11, 256, 1000, 950, 2, 0),   # q/k/v on 128 x 128 tiles
 ]
 
 
@@ -156,6 +159,54 @@ def _loop_case(cfg, seed, dv):
     cos, sin = make_rope_np(T, e.head_dim, 10_000.0, offset=valid)
     return [dv(a) for a in (rng.standard_normal(kv), rng.standard_normal(kv), rng.standard_normal((1, T, 32)), te, cos,
                             sin, make_prefix_mask_np(P, num_valid=valid))]
+
+
+def test_f32_grouped_heads():
+    """Two kv heads of two query heads each against the same model with every query head's own kv head (which
+    the oracle has): the same keys, values and loop."""
+    print("float32 grouped heads", flush=True)
+    grouped, full = _model(64, 2, 4, 2, 64, 600, 3, 3), _model(64, 2, 4, 4, 64, 600, 3, 3)
+    p = O.make_params(O.param_specs(O.dims_from_config(grouped)), 5, "float32")
+    own = {n: np.repeat(a.reshape(2, 64, -1), 2, 0).reshape(256, -1) if ".k_proj." in n or ".v_proj." in n else a
+           for n, a in p.items()}
+    out = []
+    for cfg, weights in ((grouped, p), (full, own)):
+        runner = PiZeroRunner(cfg, "rocm")
+        dv = lambda a: runtime.tensor(np.ascontiguousarray(a, np.float32), runner.dev)  # noqa: B023,E731
+        params = [dv(weights[n]) for n, _ in runner.named_params]
+        emb = dv(np.random.default_rng(1).standard_normal((1, 600, 64)))
+        args = _loop_case(grouped, 2, dv)
+        k, v = runner.vm["prefill"](emb, args[6], params)
+        x = runner.vm["denoise_loop_kv"](k, v, *args[2:], params)
+        out.append((k.numpy(), v.numpy(), x.numpy()))
+    (k, v, x), (ko, vo, xo) = out
+    _tol(np.repeat(k, 2, 2), ko, "keys")
+    _tol(np.repeat(v, 2, 2), vo, "values")
+    _tol(x, xo, "loop")
+
+
+def test_f32_replays_take_new_inputs():
+    """Replays of the loop and the chunk with another cache, noise, time embeddings, rotations, mask and prefix
+    each time, all kept alive at addresses of their own, and with other parameters bound in between, against
+    direct launches: the same bits."""
+    print("float32 replays with new inputs", flush=True)
+    cfg = _model(64, 2, 2, 1, 32, 70, 5, 3)
+    d = O.dims_from_config(cfg)
+    replayed, direct = PiZeroRunner(cfg, "rocm", cuda_graph=True), PiZeroRunner(cfg, "rocm")
+    dv = lambda a: runtime.tensor(np.ascontiguousarray(a, np.float32), direct.dev)  # noqa: E731
+    lists = [[dv(p[n]) for n, _ in direct.named_params]
+             for p in (O.make_params(O.param_specs(d), seed, "float32") for seed in (1, 2))]
+    cases = [_loop_case(cfg, seed, dv) for seed in range(7)]
+    embs = [dv(np.random.default_rng(seed).standard_normal((1, 70, 64))) for seed in range(7)]
+    seen = []
+    for i, which in enumerate((0, 0, 0, 1, 1, 0, 0)):
+        params, args, emb = lists[which], cases[i], embs[i]
+        chunk_args = (emb, args[6], *args[2:6], params)
+        for fn, a in (("denoise_loop_kv", (*args, params)), ("chunk", chunk_args)):
+            got, ref = (r.vm[fn](*a).numpy() for r in (replayed, direct))
+            np.testing.assert_array_equal(got, ref, err_msg=f"{fn}, call {i}")
+            assert all(np.abs(ref - s).max() > 1e-4 for s in seen), f"{fn}, call {i}: not new"
+            seen.append(ref)
 
 
 def test_f32_many_layers():

@@ -59,6 +59,23 @@ def test_noalloc_linear_matches_linear_twice(q4):
         assert torch.equal(y, y_ref), (y.float() - y_ref.float()).abs().max().item()
 
 
+@pytest.mark.parametrize("q4", [False, True], ids=["f16", "q4"])
+def test_noalloc_linear_scratch_twice(q4):
+    # the same over shapes whose K slices meet in the scratch (more rows x K than the few-row kernel takes): 8
+    # slices of 32 output tiles, then other tiles and slice counts over what the first call left there
+    for m, k, n in ((50, 4096, 2048), (16, 2048, 512), (64, 8192, 192)):
+        print(f"noalloc linear over the scratch M={m} K={k} N={n} q4={q4}", flush=True)
+        x, w, qw, qs, b = _case(m, k, n, q4, seed=m + k + n)
+        y_ref = torch.empty((m, n), dtype=torch.float16, device="cuda")
+        ys = [torch.full((m, n), float("nan"), dtype=torch.float16, device="cuda") for _ in range(2)]
+        N.call("mlcv_linear", _p(x), m, k, _p(w), _p(qw), _p(qs), _p(b), _p(y_ref), n, _st())
+        for y in ys:
+            N.call("mlcv_linear_noalloc", _p(x), m, k, _p(w), _p(qw), _p(qs), _p(b), _p(y), n, _st())
+        torch.cuda.synchronize()
+        for y in ys:
+            assert torch.equal(y, y_ref), (y.float() - y_ref.float()).abs().max().item()
+
+
 def test_noalloc_linear_refuses_sizes_beyond_its_scratch():
     m, k, n = 1, 32, 64 * 70000  # 70000 output tiles: more arrival counters than the scratch holds
     x = torch.zeros((m, k), dtype=torch.float16, device="cuda")
