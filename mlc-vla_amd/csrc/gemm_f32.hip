@@ -1,6 +1,6 @@
 // The float32 model's linears on the fp32 matrix cores (v_mfma_f32_32x32x2_f32 and 16x16x4: products
 // and sums in fp32, 256 flop per clock and CU, about 155 TFLOP/s), with the norm before a linear in
-// its loader and the elementwise work after it in its epilogue.
+// the same pass (few rows; many rows: a launch before it) and the elementwise work after it in its epilogue.
 //
 // Two kernels over the same operands and epilogues:
 // - f32_tile_kernel: many rows (prefill).  Workgroup tiles of 128 x 128 or 64 x 64, 4 waves in 2 x 2,
@@ -554,13 +554,27 @@ int f32_gemm_launch(const F32Op& in, hipStream_t st) {
   while (mt > 1 && (long)((a.N + 15) / 16) * ((a.M + 16 * mt - 1) / (16 * mt)) < cus) mt >>= 1;
   if (a.tab) return tab_launch(a, mt, st);
   switch (a.epi) {
-    case FE_STORE: return norm == 2 ? skinny_launch<2, FE_STORE>(a, mt, st) : norm == 1 ? skinny_launch<1, FE_STORE>(a, mt, st) : skinny_launch<0, FE_STORE>(a, mt, st);
-    case FE_QKV: return norm == 2 ? skinny_launch<2, FE_QKV>(a, mt, st) : norm == 1 ? skinny_launch<1, FE_QKV>(a, mt, st) : skinny_launch<0, FE_QKV>(a, mt, st);
-    case FE_RES: return skinny_launch<0, FE_RES>(a, mt, st);
-    case FE_GEGLU: return norm == 2 ? skinny_launch<2, FE_GEGLU>(a, mt, st) : norm == 1 ? skinny_launch<1, FE_GEGLU>(a, mt, st) : skinny_launch<0, FE_GEGLU>(a, mt, st);
-    case FE_EULER: return norm == 2 ? skinny_launch<2, FE_EULER>(a, mt, st) : skinny_launch<0, FE_EULER>(a, mt, st);
-    default: MLCV_REQUIRE(false, "float32 linear: epilogue");
+    // the pairs of norm and epilogue that the model has
+    case FE_STORE:
+      if (norm == 0) return skinny_launch<0, FE_STORE>(a, mt, st);
+      if (norm == 2) return skinny_launch<2, FE_STORE>(a, mt, st);
+      break;
+    case FE_QKV:
+      if (norm == 1) return skinny_launch<1, FE_QKV>(a, mt, st);
+      if (norm == 2) return skinny_launch<2, FE_QKV>(a, mt, st);
+      break;
+    case FE_RES:
+      if (norm == 0) return skinny_launch<0, FE_RES>(a, mt, st);
+      break;
+    case FE_GEGLU:
+      if (norm == 1) return skinny_launch<1, FE_GEGLU>(a, mt, st);
+      if (norm == 2) return skinny_launch<2, FE_GEGLU>(a, mt, st);
+      break;
+    case FE_EULER:
+      if (norm == 2) return skinny_launch<2, FE_EULER>(a, mt, st);
+      break;
   }
+  MLCV_REQUIRE(false, "float32 linear: norm and epilogue");
 }
 
 }  // namespace mlcv
