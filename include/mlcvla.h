@@ -261,7 +261,9 @@ int mlcv_q4_dequantize(const uint32_t* q_weight, const void* q_scale, void* w, i
 
 /* Linear y[M,N] = x[M,K] . W[N,K]^T (+ bias) in f16 with f32 accumulation, W
  * either f16 (w) or q4f16_1 (q_weight, q_scale) -- nn.Linear / GroupQuantizeLinear
- * (quant.py:301-325).  Runs the skinny MFMA GEMM of the denoise step. */
+ * (quant.py:301-325).  Returns after the work is done.  Few rows or short K run on one
+ * launch without split K, fp16 weights over more than 64 rows on the mid-size MFMA GEMM
+ * where that is faster, everything else on the skinny MFMA GEMM of the denoise step. */
 int mlcv_linear(const void* x, int32_t M, int32_t K, const void* w, const uint32_t* q_weight, const void* q_scale,
                 const void* bias, void* y, int32_t N, void* stream);
 

@@ -892,7 +892,7 @@ using namespace mlcv;
 
 struct mlcv_ctx {
   Ctx c;
-  F32Model* f32 = nullptr;  // a float32 model: the generic fp32 kernels of model_f32.hip
+  F32Model* f32 = nullptr;  // a float32 model (model_f32.hip)
   ~mlcv_ctx() {
     if (f32) f32_destroy(f32);
   }
@@ -2306,7 +2306,7 @@ int mlcv_embed_image(const mlcv_vision_config* cfg, const void* const* params, i
   MLCV_TRY(tile_scratch(&gws, &gsync, &gerr, &gerr_dev));
   // an earlier image whose GEMM meeting gave up is reported here (this call is not run)
   MLCV_TRY(tile_meet_failed(gerr, "an earlier mlcv_embed_image or mlcv_tile_linear call"));
-  // the ~330 launches of one image run as a hipGraph, captured on a private stream and kept
+  // the launches of one image (about 190 for the So400m tower) run as a hipGraph, captured on a private stream and kept
   // per device; a call with other pointers or another config captures again
   struct VisGraph {
     std::vector<const void*> key;
@@ -2423,11 +2423,13 @@ static bool linear_mid(const void* x, int32_t M, int32_t K, const void* w, const
 // to where its x reads (every workgroup's own, straight from the L2) outweigh the skinny kernel's staging
 // barriers and the meeting of its K slices.  From 4096 outputs on the skinny kernel's own workgroups read as
 // much of x, so the line lies higher; fp16 weights add four times the bytes of q4 to the same path, so there it
-// lies lower.  Skinny / lin_rows, us (q4; fp16), the 363 shapes measured inside are 1.01 to 4.2 times as fast:
-//   inside:  1 x 1024 x 1024  6.8 / 3.8; 6.6 / 4.2    50 x 1024 x 8192  8.8 / 6.9; 10.0 / 7.5
-//   near it: 64 x 512 x 512   5.1 / 5.0; 4.9 / 5.1    64 x 1024 x 4096  7.4 / 7.2; 7.2 / 7.6
-//   past it: 32 x 2048 x 512  6.5 / 7.6; 6.8 / 8.8    64 x 1024 x 16384 10.5 / 12.2; 12.6 / 15.1
-//            8 x 4096 x 512   8.3 / 8.9; -            968 x 256 x 1024  4.8 / 5.1; 4.5 / 5.4
+// lies lower.  Skinny / lin_rows, us; 1500 shapes measured inside are 0.99 (one of them) to 6.7 times as fast.
+//   q4    inside:  1 x 1024 x 1024 6.8 / 3.8   50 x 1024 x 8192 8.8 / 6.9   64 x 1024 x 4096 7.4 / 7.2
+//         past it: 32 x 2048 x 512 6.5 / 7.6   64 x 1024 x 16384 10.5 / 12.2   8 x 4096 x 512 8.3 / 8.9
+//                  968 x 256 x 1024 4.8 / 5.1 (two rounds)
+//   fp16  inside:  1 x 1024 x 1024 6.6 / 4.2   32 x 256 x 1024 4.8 / 2.8
+//         past it: 64 x 512 x 512 4.9 / 5.1   64 x 1024 x 4096 7.2 / 7.6   32 x 2048 x 512 6.8 / 8.8
+//                  968 x 256 x 1024 4.5 / 5.4; also, still faster, 50 x 1024 x 8192 10.0 / 7.5
 static bool linear_rows(const void* x, int32_t M, int32_t K, const void* w, const uint32_t* q_weight,
                         const void* q_scale, const void* bias, void* y, int32_t N, LinRows* a) {
   *a = LinRows{reinterpret_cast<const _Float16*>(x), M, K, N, reinterpret_cast<const _Float16*>(w), q_weight,

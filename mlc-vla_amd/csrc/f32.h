@@ -23,7 +23,8 @@ struct F32Tab {
 // y[m][n] over x [M][ldx] and weight rows of K floats.  Logical rows n come in slabs of 16: FE_GEGLU
 // pairs 8 gate rows with their 8 up rows, q and k pair dims d .. d + 7 with their RoPE partners
 // d + hd/2 .. (so a pair is 8 rows apart in one tile); the rest are in order.
-// Needs K % 8 == 0, N % 8 == 0, 16-byte aligned rows and pointers (f32_gemm_ok).
+// Needs K % 8 == 0, N % 8 == 0, ldx % 4 == 0 (checked) and 16-byte aligned pointers and output rows,
+// which the caller sees to (F32Model::fast, f32_aligned).
 struct F32Op {
   const float* x;
   int ldx, M, K, N;
@@ -33,7 +34,7 @@ struct F32Op {
   int ntab;
   size_t tab_stride;
   // x is normalised first: x / sqrt(mean(x^2) + eps), then * (1 + nw) (RMSNorm) or
-  // * (1 + mod[k]) + mod[K + k] (adaRMS); in the kernel's loader, or by a launch into xn [M][K]
+  // * (1 + mod[k]) + mod[K + k] (adaRMS); in the kernel's pass over x, or by a launch into xn [M][K]
   const float* nw;
   const float* mod;
   float eps;

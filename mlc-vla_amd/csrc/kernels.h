@@ -407,7 +407,7 @@ int euler_init_launch(const float* x0, float* x32, _Float16* x16, int n, hipStre
 // the weights of its next task before it waits for the previous phase, and the phases
 // meet through per-workgroup progress words instead of kernel boundaries.
 // ---------------------------------------------------------------------------
-// The float32 model (model_f32.hip): generic fp32 kernels for prefill / step / loop / chunk.
+// The float32 model (model_f32.hip): prefill / step / loop / chunk in fp32.
 struct F32Model;
 int f32_create(const ::mlcv_config& cfg, F32Model** out);
 void f32_destroy(F32Model* m);

@@ -133,8 +133,8 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const _Float16* __restri
 }
 
 // LayerNorm of one row per wave, the row in registers (n % 8 == 0, n <= 512 NP, 16-byte aligned): one pass
-// and no barriers.  256 rows of 1152: 3.7 us, 6.8 beside the prefetch workgroups (a block per row, two
-// passes: 4.9).
+// and no barriers.  256 rows of 1152: 4.8 us in a kernel trace, 7.7 beside the prefetch workgroups (a block per
+// row, two passes: 4.8 there, without room for them).
 template <int NP>
 __global__ __launch_bounds__(64) void layernorm_wave_kernel(const _Float16* __restrict__ x, const _Float16* __restrict__ w,
                                                             const _Float16* __restrict__ b, int n, float eps,
