@@ -156,12 +156,14 @@ static void check_mid_linear() {
       {83, 416, 15748, false},   // 9.5 / 11.2
       {968, 768, 16384, true},   // 106.8 / 78.1
       {942, 672, 2128, false},   // 14.4 / 15.9: rows across lines
+      {671, 608, 2680, true},    // 16.1 / 15.1
       {582, 928, 2908, true},    // 17.6 / 14.1
       {640, 8192, 64, true},     // 16.3 / 14.0
       {1100, 8192, 64, false},   // 19.8 / 24.3: an XCD or two
       {1226, 14112, 256, false}, // 49.1 / 57.1
       {285, 7968, 64, false},    // 14.5 / 16.4: rows across lines
       {126, 16160, 28, false},   // 21.4 / 25.3
+      {227, 9888, 8, true},      // 20.5 / 13.6
       {801, 3328, 32, true},     // 11.2 / 8.1
       {3846, 800, 2324, false},  // 55.8 / 65.0
       {16384, 512, 256, false},  // 19.5 / 42.2

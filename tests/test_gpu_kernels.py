@@ -219,7 +219,7 @@ MID_SHAPES = [(64, 512, 64, True, 0), (65, 512, 64, True, 0), (65, 256, 64, True
               (96, 544, 100, True, 0), (97, 2080, 1028, True, 0), (128, 1056, 4096, False, 0),
               (200, 320, 32, True, 4), (256, 1152, 1152, True, 0), (256, 1152, 4304, True, 0), (457, 1024, 2560, True, 0),
               (968, 512, 2052, False, 0), (1030, 16384, 16, True, 0), (968, 576, 2052, False, 0),
-              (1024, 16384, 16, True, 0), (200, 3616, 64, True, 0), (2049, 1024, 1024, False, 0)]
+              (1024, 16384, 16, True, 0), (200, 9888, 64, True, 0), (2049, 1024, 1024, False, 0)]
 
 
 @pytest.mark.parametrize("noalloc", [False, True], ids=["linear", "noalloc"])
