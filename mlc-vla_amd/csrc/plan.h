@@ -149,13 +149,13 @@ inline bool mid_vs_tile(int M, int N, int K, int cus) {
 
 // fp16 linears (mlcv_linear) that run on this kernel, not on the skinny one: the shapes of more than 64
 // rows and K > 256 where it is the faster of the two.  Kernel times over 2800 shapes of 65 to 16384 rows on
-// 256 CUs, skinny / this, us; inside it is 0.97 to 4 times as fast.
+// 256 CUs, skinny / this, us; inside it is 0.95 to 4 times as fast.
 // - One round of tiles: 100 x 2048 x 2048 9.7 / 6.1, 457 x 2048 x 2560 30.4 / 14.3, 256 x 512 x 4096 7.6 / 6.4.
 //   Few outputs are a few n tiles, whose m tiles share an XCD each, while the skinny kernel splits K: past
 //   1024 rows 1100 x 8192 x 64 19.8 / 24.3, 1226 x 14112 x 256 49.1 / 57.1.  Rows that straddle 128-byte lines
-//   (K % 64 = 32) cost a wave two lines a row and stage; with few outputs that loses at K up to 8192, where the
-//   skinny kernel's 8 slices grow from 1024 k, and near 16384: 285 x 7968 x 64 14.5 / 16.4, 126 x 16160 x 28 21.4 /
-//   25.3, but 227 x 9888 x 8 20.5 / 13.6.  At 4096 the two are about even: 956 x 4064 x 56 12.5 / 12.8.
+//   (K % 64 = 32) cost a wave two lines a row and stage; with few outputs that loses at K just below 8192
+//   and near 16384: 285 x 7968 x 64 14.5 / 16.4, 126 x 16160 x 28 21.4 / 25.3, but 227 x 9888 x 8 20.5 / 13.6.
+//   Just below 4096 the two are about even: 956 x 4064 x 56 12.5 / 12.8.
 // - More rounds: up to K = 512 968 x 512 x 4096 17.6 / 20.4, 457 x 288 x 16384 26.0 / 35.8; past it 968 x
 //   768 x 16384 106.8 / 78.1, 671 x 608 x 2680 16.1 / 15.1.  More than 900 straddling rows: 942 x 672 x 2128 14.4 /
 //   15.9, from K = 800 on faster.  Past 2048 rows or below 1024 outputs: 3846 x 800 x 2324 55.8 / 65.0, 16384 x
